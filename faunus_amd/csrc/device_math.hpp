@@ -28,6 +28,18 @@ __device__ __forceinline__ double dist2(const Box& b, double ax, double ay, doub
     return dx * dx + dy * dy + dz * dz;
 }
 
+// Squared distance to the nearest image by rounding: at most that of dist2 (equal to it up
+// to rounding for coordinates inside the box) in half its instructions, to tell far pairs
+// from near ones before dist2 is taken.
+__device__ __forceinline__ double near_dist2(const Box& b, const double inv[3], double ax, double ay, double az,
+                                             double bx, double by, double bz) {
+    double dx = ax - bx, dy = ay - by, dz = az - bz;
+    dx = fma(-b.L[0], rint(dx * inv[0]), dx);
+    dy = fma(-b.L[1], rint(dy * inv[1]), dy);
+    dz = fma(-b.L[2], rint(dz * inv[2]), dz);
+    return dx * dx + dy * dy + dz * dz;
+}
+
 // tabulate.h:184-202: interval by lower_bound, Horner from the top coefficient.  The
 // lower_bound starts one knot before the first knot of x's uniform bucket and takes a
 // fixed number of compare-and-step rounds (enough for the fullest bucket), which finds

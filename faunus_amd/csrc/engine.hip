@@ -379,97 +379,204 @@ __global__ void commit_kernel(double4* pos, MoveArgs mv, CellArgs cells, int* ce
     }
 }
 
-// Full structure factors Q(k) = sum_j q_j e^{ik.r_j} (energy.cpp:191-206); particle
-// order as in the reference (groups in order, particles in order).
-__global__ __launch_bounds__(kBlock) void full_q_kernel(const double4* __restrict__ pos, int n,
-                                                         const int* __restrict__ kn, int nk, Box box,
-                                                         double2* __restrict__ q_out) {
-    __shared__ double4 tile[kBlock];
-    const int k = blockIdx.x * kBlock + threadIdx.x;
+// Full structure factors Q(k) = sum_j q_j e^{ik.r_j} (energy.cpp:191-206) as a matrix
+// product.  A column is one (nx, ny); with B_j = q_j e^{i kx xj} e^{i ky yj} the row sums
+//   R = sum_j Re(B_j) {cos, sin}(kz zj),  I = sum_j Im(B_j) {cos, sin}(kz zj)
+// give Q at +nz and -nz, so the work is a real product of [2 x columns, particles] by
+// [particles, 2 (ncut + 1)]: two multiply-adds per k-vector and particle, and 3 (ncut + 1)
+// sincos per particle and block in place of one sincos per k-vector and particle.
+// A block takes kQCols x kCT columns (16 per wave and tile) and a slice of the particles;
+// per chunk it writes the particles' axis tables to LDS, from which each wave forms its A
+// operands (lane: column l mod 16, particle l div 16) and reads its B operands.  Columns
+// are sorted by their largest nz, so that a wave's tiles skip the nz no column of it has.
+// The slices' partial Q(k) are added in slice order by sum_q_kernel.
+// N = 20000, K = 17328: 4455 us with one thread per k-vector and a sincos per particle (68
+// blocks, latency bound), now 95 + 7 us (the products and the tables' sincos);
+// N = 12288, K = 1661: 2784 -> 20 + 12 us.
+constexpr int kQThreads = 512;
+constexpr int kQCols = 16 * kQThreads / 64; // columns per block and column tile
+constexpr int kQTiles = 3;                  // 16-wide tiles of (cos, sin) x nz per wave
+constexpr int kQChunk = 32;                 // particles per LDS chunk, at most
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+template <int kCT>
+__global__ __launch_bounds__(kQThreads) void full_q_kernel(const double4* __restrict__ pos, int n,
+                                                           const QColumn* __restrict__ cols, int ncol, int ncut,
+                                                           int chunk, int slice, int nk, Box box,
+                                                           double2* __restrict__ partial) {
+    extern __shared__ double2 s_tab[]; // [chunk][3][ncut + 1], the x table times the charge
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int w = ncut + 1, row = 3 * w;
     const double twopi = 6.283185307179586;
-    double kx = 0, ky = 0, kz = 0;
-    if (k < nk) {
-        const int packed = kn[k];
-        kx = twopi * (static_cast<double>(unpack_n(packed, 0)) / box.L[0]);
-        ky = twopi * (static_cast<double>(unpack_n(packed, 1)) / box.L[1]);
-        kz = twopi * (static_cast<double>(unpack_n(packed, 2)) / box.L[2]);
+    const int c0 = kQTiles * 16 * static_cast<int>(blockIdx.z); // first (cos, sin) x nz entry of this block
+    int nx[kCT], ny[kCT], tiles[kCT];
+    double sy[kCT];
+    f64x4 re[kCT][kQTiles], im[kCT][kQTiles];
+    const int first = (static_cast<int>(blockIdx.x) * kCT * (kQThreads / 64) + wave * kCT) * 16;
+#pragma unroll
+    for (int ct = 0; ct < kCT; ++ct) {
+        const int base = first + 16 * ct;
+        const QColumn c = cols[min(base + (lane & 15), ncol - 1)];
+        nx[ct] = c.nx;
+        ny[ct] = c.ny < 0 ? -c.ny : c.ny;
+        sy[ct] = c.ny < 0 ? -1.0 : 1.0;
+        // the first column of a tile has its largest nz
+        const int top = base < ncol ? 2 * (cols[base].nzmax + 1) - c0 : 0;
+        tiles[ct] = __builtin_amdgcn_readfirstlane(top <= 0 ? 0 : min(kQTiles, (top + 15) / 16));
+#pragma unroll
+        for (int t = 0; t < kQTiles; ++t) re[ct][t] = im[ct][t] = f64x4{0.0, 0.0, 0.0, 0.0};
     }
-    double re = 0.0, im = 0.0;
-    for (int base = 0; base < n; base += kBlock) {
-        __syncthreads();
-        if (base + threadIdx.x < static_cast<unsigned>(n)) tile[threadIdx.x] = pos[base + threadIdx.x];
-        __syncthreads();
-        const int cnt = min(kBlock, n - base);
-        if (k < nk) {
-            for (int j = 0; j < cnt; ++j) {
-                const double4 p = tile[j];
+    const int j1 = min(n, slice * (static_cast<int>(blockIdx.y) + 1));
+    for (int base = slice * static_cast<int>(blockIdx.y); base < j1; base += chunk) {
+        __syncthreads(); // the previous chunk's tables are consumed
+        for (int e = tid; e < chunk * row; e += kQThreads) {
+            const int j = e / row, r = e - j * row, axis = r / w;
+            double2 v = make_double2(0.0, 0.0);
+            if (base + j < j1) {
+                const double4 p = pos[base + j];
+                const double x = axis == 0 ? p.x : (axis == 1 ? p.y : p.z);
                 double sn, cs;
-                sincos(kx * p.x + ky * p.y + kz * p.z, &sn, &cs);
-                re += p.w * cs;
-                im += p.w * sn;
+                sincos(twopi * (static_cast<double>(r - axis * w) / box.L[axis]) * x, &sn, &cs);
+                v = axis == 0 ? make_double2(p.w * cs, p.w * sn) : make_double2(cs, sn);
+            }
+            s_tab[e] = v;
+        }
+        __syncthreads();
+        for (int p = 0; p < chunk; p += 4) {
+            const double2* tab = s_tab + (p + (lane >> 4)) * row;
+            // entries past 2 (ncut + 1) belong to unused output columns: the next particle's
+            // table, or the pad behind the last one
+            const double* zt = reinterpret_cast<const double*>(tab + 2 * w) + c0 + (lane & 15);
+            double bz[kQTiles];
+#pragma unroll
+            for (int t = 0; t < kQTiles; ++t) bz[t] = zt[16 * t];
+#pragma unroll
+            for (int ct = 0; ct < kCT; ++ct) {
+                if (tiles[ct] == 0) continue;
+                const double2 X = tab[nx[ct]], Y = tab[w + ny[ct]];
+                const double yi = sy[ct] * Y.y;
+                const double ar = X.x * Y.x - X.y * yi, ai = X.x * yi + X.y * Y.x;
+#pragma unroll
+                for (int t = 0; t < kQTiles; ++t)
+                    if (t < tiles[ct]) {
+                        re[ct][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, bz[t], re[ct][t], 0, 0, 0);
+                        im[ct][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, bz[t], im[ct][t], 0, 0, 0);
+                    }
             }
         }
     }
-    if (k < nk) q_out[k] = make_double2(re, im);
+    // even lanes hold the cos sums of an nz and write Q(+nz), odd lanes its sin sums and
+    // write Q(-nz); the partner's sums come by a pair swap.  Element r of lane l is column
+    // 4 r + l div 16 of the tile, entry l mod 16.
+    double2* out = partial + static_cast<size_t>(blockIdx.y) * static_cast<size_t>(nk);
+#pragma unroll
+    for (int ct = 0; ct < kCT; ++ct)
+#pragma unroll
+        for (int t = 0; t < kQTiles; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const double a = re[ct][t][r], b = im[ct][t][r];
+                const double a2 = __builtin_amdgcn_update_dpp(0.0, a, 0xB1, 0xF, 0xF, false);
+                const double b2 = __builtin_amdgcn_update_dpp(0.0, b, 0xB1, 0xF, 0xF, false);
+                const int col = first + 16 * ct + 4 * r + (lane >> 4);
+                const int nz = (c0 + 16 * t + (lane & 15)) >> 1;
+                const bool odd = lane & 1;
+                if (t >= tiles[ct] || col >= ncol || (odd && nz == 0)) continue;
+                const QColumn c = cols[col];
+                const int z = odd ? -nz : nz;
+                const bool hole = c.nx == 0 && c.ny == 0; // k = 0 is left out
+                if (z < c.nzmin || z > c.nzmax || (hole && z == 0)) continue;
+                out[c.k0 + (z - c.nzmin) - (hole && z > 0 ? 1 : 0)] =
+                    odd ? make_double2(a2 + b, b2 - a) : make_double2(a - b2, a2 + b);
+            }
 }
 
-// All pairs i<j (Change::everything, energy.h:1290-1299): one thread per i, j>i.
-template <bool kGroups>
+// Sum of the slices' partial structure factors, in slice order.
+__global__ __launch_bounds__(kBlock) void sum_q_kernel(const double2* __restrict__ partial, int slices, int nk,
+                                                       double2* __restrict__ q_out) {
+    const int k = blockIdx.x * kBlock + threadIdx.x;
+    if (k >= nk) return;
+    double2 s = partial[k];
+#pragma unroll 8
+    for (int i = 1; i < slices; ++i) {
+        const double2 v = partial[static_cast<size_t>(i) * static_cast<size_t>(nk) + static_cast<size_t>(k)];
+        s.x += v.x;
+        s.y += v.y;
+    }
+    q_out[k] = s;
+}
+
+// All pairs i < j (Change::everything, energy.h:1290-1299).  Block (x, y) pairs the
+// particles i of tile x (one per thread) with those of run y of `len` particles; j is the
+// same for every lane, so its coordinates come through scalar loads.  kCut: every pair
+// energy is exactly zero beyond a distance, and `range2` lies just above its square; a wave
+// whose 64 pairs are all farther goes on after the rounded distance.
+// One block per tile over all later particles (79 blocks of up to 20000 steps, one wave
+// per SIMD) took 5848 us at N = 20000 with the pair energy cut at 12 A, now 178 us; 4096
+// waters with a group cutoff took 12528 us, now 521.
+template <bool kGroups, bool kCut>
 __global__ __launch_bounds__(kBlock) void all_pairs_kernel(const double4* __restrict__ pos,
                                                             const uint32_t* __restrict__ meta, int n,
                                                             const DevPair* __restrict__ pairs_g, int ntypes,
                                                             const DevCoulomb* __restrict__ coul_g, Box box,
-                                                            GroupTable groups, double* __restrict__ partials) {
+                                                            GroupTable groups, int len, double range2,
+                                                            double* __restrict__ partials) {
     __shared__ DevPair s_pairs[kMaxTypes * kMaxTypes];
     __shared__ DevCoulomb s_coul;
-    __shared__ double4 tile[kBlock];
-    __shared__ uint32_t tmeta[kBlock];
     __shared__ double s_red[kBlock / 64];
+    const int part = static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
+    const int i0 = static_cast<int>(blockIdx.x) * kBlock, jb = static_cast<int>(blockIdx.y) * len;
+    const int je = min(n, jb + len);
+    if (je <= i0 + 1) { // no j of this run is behind an i of this tile
+        if (threadIdx.x == 0) partials[part] = 0.0;
+        return;
+    }
     for (int i = threadIdx.x; i < ntypes * ntypes; i += kBlock) s_pairs[i] = pairs_g[i];
     lds_copy(s_coul, coul_g, static_cast<int>(threadIdx.x), kBlock);
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    double4 pi = make_double4(0, 0, 0, 0);
-    uint32_t mi = 0;
-    if (i < n) {
-        pi = pos[i];
-        mi = meta[i];
-    }
+    const int i = i0 + static_cast<int>(threadIdx.x);
+    const double4 pi = pos[min(i, n - 1)];
+    const uint32_t mi = meta[min(i, n - 1)];
     const int ti = static_cast<int>(mi & 0xffu), gi = static_cast<int>(mi >> 8);
+    __syncthreads();
+    const double inv[3] = {1.0 / box.L[0], 1.0 / box.L[1], 1.0 / box.L[2]};
     double acc = 0.0;
-    for (int base = blockIdx.x * kBlock; base < n; base += kBlock) {
-        __syncthreads();
-        if (base + threadIdx.x < static_cast<unsigned>(n)) {
-            tile[threadIdx.x] = pos[base + threadIdx.x];
-            tmeta[threadIdx.x] = meta[base + threadIdx.x];
-        }
-        __syncthreads();
-        const int cnt = min(kBlock, n - base);
-        if (i < n) {
-            for (int jj = 0; jj < cnt; ++jj) {
-                const int j = base + jj;
-                if (j <= i) continue;
-                const uint32_t mj = tmeta[jj];
-                const int gj = static_cast<int>(mj >> 8);
-                if (kGroups) {
-                    if (gi == gj) {
-                        if (groups.flags[gi] & 2) continue; // rigid: no internal pairs
-                        if (pair_excluded(groups.excl_off, groups.excl, i, j)) continue;
-                    } else if (groups.g2g2 && (groups.flags[gi] & 1) && (groups.flags[gj] & 1)) {
-                        const double* a = groups.cm + 3 * gi;
-                        const double* b = groups.cm + 3 * gj;
-                        if (!(dist2(box, a[0], a[1], a[2], b[0], b[1], b[2]) <
-                              g2g_cutoff2(groups.g2g2, groups.nmol, groups.flags[gi], groups.flags[gj])))
-                            continue;
-                    }
-                }
-                const double4 pj = tile[jj];
-                const DevPair& p = s_pairs[ti * ntypes + static_cast<int>(mj & 0xffu)];
-                acc += pair_energy(p, s_coul, pi.w, pj.w, dist2(box, pi.x, pi.y, pi.z, pj.x, pj.y, pj.z));
+#pragma unroll 2
+    for (int j = max(jb, i0 + 1); j < je; ++j) {
+        const double4 pj = pos[j];
+        if (kCut && near_dist2(box, inv, pi.x, pi.y, pi.z, pj.x, pj.y, pj.z) >= range2) continue;
+        if (j <= i || i >= n) continue;
+        const double r2 = dist2(box, pi.x, pi.y, pi.z, pj.x, pj.y, pj.z);
+        const uint32_t mj = meta[j];
+        if (kGroups) {
+            const int gj = static_cast<int>(mj >> 8);
+            if (gi == gj) {
+                if (groups.flags[gi] & 2) continue; // rigid: no internal pairs
+                if (pair_excluded(groups.excl_off, groups.excl, i, j)) continue;
+            } else if (groups.g2g2 && (groups.flags[gi] & 1) && (groups.flags[gj] & 1)) {
+                const double* a = groups.cm + 3 * gi;
+                const double* b = groups.cm + 3 * gj;
+                if (!(dist2(box, a[0], a[1], a[2], b[0], b[1], b[2]) <
+                      g2g_cutoff2(groups.g2g2, groups.nmol, groups.flags[gi], groups.flags[gj])))
+                    continue;
             }
         }
+        const DevPair& p = s_pairs[ti * ntypes + static_cast<int>(mj & 0xffu)];
+        acc += pair_energy(p, s_coul, pi.w, pj.w, r2);
     }
     const double s = block_sum<kBlock>(acc, s_red);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
+    if (threadIdx.x == 0) partials[part] = s;
+}
+
+// Sum of `count` partials in a fixed order (one block).
+__global__ __launch_bounds__(kBlock) void sum_partials_kernel(const double* __restrict__ partials, int count,
+                                                               double* __restrict__ out) {
+    __shared__ double s_red[kBlock / 64];
+    double acc = 0.0;
+#pragma unroll 4
+    for (int b = threadIdx.x; b < count; b += kBlock) acc += partials[b];
+    const double s = block_sum<kBlock>(acc, s_red);
+    if (threadIdx.x == 0) *out = s;
 }
 
 // Plain streaming copy of a known byte count; its HBM counter readings calibrate
@@ -553,6 +660,7 @@ Engine::~Engine() {
     (void)hipFree(d_pairs_);
     (void)hipFree(d_coul_);
     (void)hipFree(d_kn_);
+    (void)hipFree(d_qcol_);
     (void)hipFree(d_ak_);
     (void)hipFree(d_q_acc_);
     (void)hipFree(d_q_trial_);
@@ -842,6 +950,21 @@ void Engine::build_kvectors() {
                 ak.push_back((nx > 0 ? 2.0 : 1.0) * std::exp(-k2 / (4 * e.alpha * e.alpha)) / k2);
             }
     nk_ = static_cast<int>(kn.size());
+    // the (nx, ny) columns of the list: each a run of k-vectors with nz ascending
+    std::vector<QColumn> cols;
+    for (int k = 0; k < nk_; ++k) {
+        const int nx = static_cast<signed char>(kn[static_cast<size_t>(k)] & 0xff);
+        const int ny = static_cast<signed char>((kn[static_cast<size_t>(k)] >> 8) & 0xff);
+        const int nz = static_cast<signed char>((kn[static_cast<size_t>(k)] >> 16) & 0xff);
+        if (cols.empty() || cols.back().nx != nx || cols.back().ny != ny)
+            cols.push_back(QColumn{static_cast<short>(nx), static_cast<short>(ny), k, nz, nz});
+        cols.back().nzmax = nz;
+    }
+    std::stable_sort(cols.begin(), cols.end(), [](const QColumn& a, const QColumn& b) { return a.nzmax > b.nzmax; });
+    ncol_ = static_cast<int>(cols.size());
+    check_hip(hipMalloc(&d_qcol_, sizeof(QColumn) * std::max(1, ncol_)), "hipMalloc k columns");
+    if (ncol_ > 0)
+        check_hip(hipMemcpy(d_qcol_, cols.data(), sizeof(QColumn) * cols.size(), hipMemcpyHostToDevice), "copy k columns");
     check_hip(hipMalloc(&d_kn_, sizeof(int) * std::max(1, nk_)), "hipMalloc kn");
     check_hip(hipMalloc(&d_ak_, sizeof(double) * std::max(1, nk_)), "hipMalloc ak");
     check_hip(hipMalloc(&d_q_acc_, sizeof(double2) * std::max(1, nk_)), "hipMalloc q");
@@ -861,12 +984,43 @@ static Box make_box(const Model& m) {
     return b;
 }
 
+// Full Q(k) from the positions into `out`; complete when it returns.
 void Engine::full_q(double2* out) {
     if (nk_ == 0) return;
     const Box box = make_box(model_);
-    hipLaunchKernelGGL(full_q_kernel, dim3((nk_ + kBlock - 1) / kBlock), dim3(kBlock), 0, stream_, d_pos_, n_, d_kn_,
-                       nk_, box, out);
-    check_hip(hipGetLastError(), "full_q_kernel");
+    const int ncut = static_cast<int>(std::ceil(model_.ewald.n_cutoff));
+    // two column tiles per wave once one would take a second block of columns (a block's
+    // table sincos then serve twice the columns)
+    const int ct = ncol_ > kQCols ? 2 : 1;
+    const int col_blocks = (ncol_ + kQCols * ct - 1) / (kQCols * ct);
+    const int z_blocks = (2 * (ncut + 1) + 16 * kQTiles - 1) / (16 * kQTiles);
+    const size_t row = sizeof(double2) * 3 * static_cast<size_t>(ncut + 1);
+    int chunk = kQChunk;
+    while (chunk > 4 && chunk * row > 40 * 1024) chunk /= 2;
+    // slices of the particles: one block per CU, or as many as there are chunks or as fit
+    // 24 MB of partial sums
+    int slices = std::max(1, num_cu_ / (col_blocks * z_blocks));
+    slices = std::min({slices, (n_ + chunk - 1) / chunk,
+                       std::max(1, static_cast<int>((24u << 20) / (sizeof(double2) * static_cast<size_t>(nk_))))});
+    int slice = (n_ + slices - 1) / slices;
+    slice = (slice + chunk - 1) / chunk * chunk;
+    slices = (n_ + slice - 1) / slice;
+    double2* part = out;
+    if (slices > 1) check_hip(hipMalloc(&part, sizeof(double2) * static_cast<size_t>(slices) * static_cast<size_t>(nk_)), "hipMalloc partial Q");
+    // the pad takes the reads past the last table row (see full_q_kernel)
+    const size_t lds = chunk * row + sizeof(double) * 16 * kQTiles * static_cast<size_t>(z_blocks);
+    const dim3 grid(static_cast<unsigned>(col_blocks), static_cast<unsigned>(slices), static_cast<unsigned>(z_blocks));
+    hipLaunchKernelGGL(ct == 2 ? full_q_kernel<2> : full_q_kernel<1>, grid, dim3(kQThreads), lds, stream_, d_pos_, n_,
+                       d_qcol_, ncol_, ncut, chunk, slice, nk_, box, part);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && slices > 1) {
+        hipLaunchKernelGGL(sum_q_kernel, dim3((nk_ + kBlock - 1) / kBlock), dim3(kBlock), 0, stream_, part, slices, nk_, out);
+        e = hipGetLastError();
+    }
+    const hipError_t done = hipStreamSynchronize(stream_);
+    if (part != out) (void)hipFree(part);
+    check_hip(e, "full_q_kernel");
+    check_hip(done, "full Q");
 }
 
 void Engine::set_cell_capacity(int cap) {
@@ -993,7 +1147,6 @@ void Engine::init() {
     if (model_.ewald.present) {
         build_kvectors();
         full_q(d_q_acc_);
-        check_hip(hipStreamSynchronize(stream_), "init full Q");
     }
     for (int d = 0; d < 3; ++d) {
         dipole_[d] = 0;
@@ -1278,32 +1431,50 @@ void Engine::total_energy(double* terms) {
             self += gs;
         }
     }
-    // nonbonded: all pairs (GroupPairing::all, energy.h:1290-1299)
-    const int blocks = (n_ + kBlock - 1) / kBlock;
+    // nonbonded: all pairs (GroupPairing::all, energy.h:1290-1299).  The runs of j are cut
+    // shorter, down to 16, until there are about eight blocks per CU
+    const int tiles = (n_ + kBlock - 1) / kBlock;
+    int len = kBlock;
+    while (len > 16 && static_cast<long long>(tiles) * ((n_ + len - 1) / len) < 16LL * num_cu_) len /= 2;
+    while (static_cast<long long>(tiles) * ((n_ + len - 1) / len) > (1LL << 17)) len *= 2;
+    const int runs = (n_ + len - 1) / len;
+    const int blocks = tiles * runs;
+    // pairs from the range on add exactly zero; 1e-9 above its square for rounding
+    const double range = model_.pair_range;
+    const double range2 = std::isfinite(range) ? range * range * (1.0 + 1e-9) : kInf;
     const int bond_blocks = nbonds_ > 0 ? std::min(64, (nbonds_ + kBlock - 1) / kBlock) : 0;
-    double* d_part = nullptr;
-    check_hip(hipMalloc(&d_part, sizeof(double) * (blocks + bond_blocks)), "hipMalloc partials");
-    GroupTable gt{d_gflags_, d_gcm_, d_g2g_, static_cast<int>(model_.molecules.size()), d_excl_off_, d_excl_};
-    if (any_molecular_)
-        hipLaunchKernelGGL((all_pairs_kernel<true>), dim3(blocks), dim3(kBlock), 0, stream_, d_pos_, d_meta_, n_,
-                           d_pairs_, model_.ntypes, d_coul_, make_box(model_), gt, d_part);
-    else
-        hipLaunchKernelGGL((all_pairs_kernel<false>), dim3(blocks), dim3(kBlock), 0, stream_, d_pos_, d_meta_, n_,
-                           d_pairs_, model_.ntypes, d_coul_, make_box(model_), gt, d_part);
-    check_hip(hipGetLastError(), "all_pairs_kernel");
-    if (bond_blocks > 0) {
-        hipLaunchKernelGGL(bond_total_kernel, dim3(bond_blocks), dim3(kBlock), 0, stream_, d_pos_, d_bond_all_, nbonds_,
-                           make_box(model_), d_part + blocks);
-        check_hip(hipGetLastError(), "bond_total_kernel");
+    double* d_part = nullptr; // pair partials, bond partials, pair sum, bond sum
+    check_hip(hipMalloc(&d_part, sizeof(double) * (static_cast<size_t>(blocks + bond_blocks) + 2)), "hipMalloc partials");
+    double* d_sum = d_part + blocks + bond_blocks;
+    double sums[2] = {0.0, 0.0};
+    try {
+        GroupTable gt{d_gflags_, d_gcm_, d_g2g_, static_cast<int>(model_.molecules.size()), d_excl_off_, d_excl_};
+        const auto kernel = any_molecular_ ? (range2 < kInf ? all_pairs_kernel<true, true> : all_pairs_kernel<true, false>)
+                                           : (range2 < kInf ? all_pairs_kernel<false, true> : all_pairs_kernel<false, false>);
+        hipLaunchKernelGGL(kernel,
+                           dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(runs)), dim3(kBlock), 0, stream_,
+                           d_pos_, d_meta_, n_, d_pairs_, model_.ntypes, d_coul_, make_box(model_), gt, len, range2, d_part);
+        check_hip(hipGetLastError(), "all_pairs_kernel");
+        hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kBlock), 0, stream_, d_part, blocks, d_sum);
+        check_hip(hipGetLastError(), "sum_partials_kernel");
+        if (bond_blocks > 0) {
+            hipLaunchKernelGGL(bond_total_kernel, dim3(bond_blocks), dim3(kBlock), 0, stream_, d_pos_, d_bond_all_,
+                               nbonds_, make_box(model_), d_part + blocks);
+            check_hip(hipGetLastError(), "bond_total_kernel");
+            hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kBlock), 0, stream_, d_part + blocks, bond_blocks,
+                               d_sum + 1);
+            check_hip(hipGetLastError(), "sum_partials_kernel");
+        }
+        check_hip(hipMemcpyAsync(sums, d_sum, sizeof(double) * (bond_blocks > 0 ? 2 : 1), hipMemcpyDeviceToHost, stream_),
+                  "copy sums");
+        check_hip(hipStreamSynchronize(stream_), "sync");
+    } catch (...) {
+        (void)hipStreamSynchronize(stream_);
+        (void)hipFree(d_part);
+        throw;
     }
-    std::vector<double> part(static_cast<size_t>(blocks + bond_blocks));
-    check_hip(hipMemcpyAsync(part.data(), d_part, sizeof(double) * part.size(), hipMemcpyDeviceToHost, stream_),
-              "copy partials");
-    check_hip(hipStreamSynchronize(stream_), "sync");
     (void)hipFree(d_part);
-    double pair = 0, bond = 0;
-    for (int b = 0; b < blocks; ++b) pair += part[static_cast<size_t>(b)];
-    for (int b = 0; b < bond_blocks; ++b) bond += part[static_cast<size_t>(blocks + b)];
+    const double pair = sums[0], bond = sums[1];
     double ewald = 0;
     if (model_.ewald.present) {
         std::vector<double2> q(static_cast<size_t>(nk_));
@@ -1368,7 +1539,6 @@ void Engine::reset_positions(const double* xyz, const double* mass_center) {
     }
     if (model_.ewald.present) {
         full_q(d_q_acc_);
-        check_hip(hipStreamSynchronize(stream_), "full Q");
     }
     (void)hipFree(cells_.count);
     (void)hipFree(cells_.members);

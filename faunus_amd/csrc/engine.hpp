@@ -93,6 +93,13 @@ struct DevBondPair {
     double half_k, req;
 };
 
+// One (nx, ny) column of the k-vector list: the k-vectors k0, k0 + 1, ... with nz from
+// nzmin to nzmax (without nz = 0 in the column nx = ny = 0).
+struct QColumn {
+    short nx, ny;
+    int k0, nzmin, nzmax;
+};
+
 struct CellList {
     bool enabled = false;
     int nc[3] = {0, 0, 0};
@@ -228,6 +235,8 @@ class Engine {
     DevCoulomb* d_coul_ = nullptr;
     // Ewald
     int* d_kn_ = nullptr;      // packed (nx, ny, nz) as signed bytes
+    QColumn* d_qcol_ = nullptr; // its (nx, ny) columns, longest first
+    int ncol_ = 0;
     double* d_ak_ = nullptr;
     double2* d_q_acc_ = nullptr;
     double2* d_q_trial_ = nullptr;
