@@ -491,29 +491,37 @@ void dispatch_cells(bool cells, bool f32, int grid, size_t lds, hipStream_t st, 
 // Pair-distance histogram of one configuration (AtomRDF::_sample, analysis.cpp:1556-1600):
 // types a != b: every (a, b) pair; a == b: pairs i < j.  r = |minimum-image distance|,
 // bin floor(r / dr) as Equidistant2DTable::to_bin (equidistant_table.h:32-39), bins >= nbins
-// dropped.  Block b takes particles i = b, b + grid, ...; its lanes stride over j; counts
-// go to an LDS histogram, then once per block to the global one.
+// dropped.  Block (x, y): one j per thread from `ids` (the particles of type b, `nb` of
+// them), against the i of type a in run y of `len` particles, whose coordinates are the
+// same for every lane (scalar loads).  Pairs beyond the last bin (range2: 1e-9 above its
+// squared edge) stop at the rounded distance; counts go to an LDS histogram, then once
+// per block to the global one.  N = 20000, 240 bins of 0.1 A: 717 us with one i per block
+// (every block read all positions), now 125 us.
 __global__ __launch_bounds__(256) void rdf_kernel(const double4* __restrict__ pos, const uint32_t* __restrict__ meta,
                                                   int n, int ta, int tb, double L, double half, double inv_dr,
-                                                  int nbins, unsigned long long* __restrict__ counts) {
+                                                  double range2, int nbins, int len, const int* __restrict__ ids, int nb,
+                                                  unsigned long long* __restrict__ counts) {
     extern __shared__ unsigned int s_hist[];
     for (int b = threadIdx.x; b < nbins; b += blockDim.x) s_hist[b] = 0u;
+    const int t = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    const int j = t < nb ? ids[t] : -1;
+    const double4 pj = pos[max(j, 0)];
+    const Box box{{L, L, L}, {half, half, half}};
+    const double inv[3] = {1.0 / L, 1.0 / L, 1.0 / L};
     __syncthreads();
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
-        const int ti = static_cast<int>(meta[i] & 0xffu);
-        if (ti != ta) continue; // uniform over the block
+    const int ie = min(n, len * (static_cast<int>(blockIdx.y) + 1));
+    for (int i = len * static_cast<int>(blockIdx.y); i < ie; ++i) {
+        if (static_cast<int>(meta[i] & 0xffu) != ta) continue; // uniform over the block
         const double4 pi = pos[i];
-        for (int j = (ta == tb ? i + 1 : 0) + static_cast<int>(threadIdx.x); j < n; j += blockDim.x) {
-            if (static_cast<int>(meta[j] & 0xffu) != tb) continue;
-            const double4 pj = pos[j];
-            const double dx = min_image(pi.x - pj.x, L, half);
-            const double dy = min_image(pi.y - pj.y, L, half);
-            const double dz = min_image(pi.z - pj.z, L, half);
-            // x^2 + y^2 + z^2 rounded term by term, as the reference's norm
-            const double r = sqrt(__dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz)));
-            const double x = floor(__dmul_rn(r, inv_dr));
-            if (x < static_cast<double>(nbins)) atomicAdd(&s_hist[static_cast<int>(x)], 1u);
-        }
+        if (near_dist2(box, inv, pi.x, pi.y, pi.z, pj.x, pj.y, pj.z) >= range2) continue;
+        if (j < 0 || (ta == tb && j <= i)) continue;
+        const double dx = min_image(pi.x - pj.x, L, half);
+        const double dy = min_image(pi.y - pj.y, L, half);
+        const double dz = min_image(pi.z - pj.z, L, half);
+        // x^2 + y^2 + z^2 rounded term by term, as the reference's norm
+        const double r = sqrt(__dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz)));
+        const double x = floor(__dmul_rn(r, inv_dr));
+        if (x < static_cast<double>(nbins)) atomicAdd(&s_hist[static_cast<int>(x)], 1u);
     }
     __syncthreads();
     for (int b = threadIdx.x; b < nbins; b += blockDim.x)
@@ -991,25 +999,42 @@ void Batch::rdf(int r, int type_a, int type_b, double dr, int nbins, unsigned lo
     const ReplicaState& h = h_states_[static_cast<size_t>(r)];
     if (type_a < 0 || type_b < 0 || type_a >= h.ntypes || type_b >= h.ntypes) throw std::runtime_error("rdf: bad atom type");
     if (!finalized_) finalize();
-    unsigned long long* d_counts = nullptr;
-    check_hip(hipMalloc(&d_counts, sizeof(unsigned long long) * static_cast<size_t>(nbins)), "hipMalloc rdf");
+    // the particles of type b, then the counts, in one allocation
+    std::vector<int> ids;
+    const auto& types = engines_[static_cast<size_t>(r)]->host_types();
+    for (int j = 0; j < h.n; ++j)
+        if (types[static_cast<size_t>(j)] == type_b) ids.push_back(j);
+    if (ids.empty()) return;
+    const int nb = static_cast<int>(ids.size());
+    const size_t head = (sizeof(int) * ids.size() + 7) & ~static_cast<size_t>(7);
+    unsigned char* d = nullptr;
+    check_hip(hipMalloc(&d, head + sizeof(unsigned long long) * static_cast<size_t>(nbins)), "hipMalloc rdf");
+    unsigned long long* d_counts = reinterpret_cast<unsigned long long*>(d + head);
     std::vector<unsigned long long> part(static_cast<size_t>(nbins));
     try {
+        check_hip(hipMemcpyAsync(d, ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice, stream_), "copy rdf ids");
         check_hip(hipMemsetAsync(d_counts, 0, sizeof(unsigned long long) * static_cast<size_t>(nbins), stream_),
                   "clear rdf");
-        const int grid = std::max(1, std::min(h.n, 2048));
-        hipLaunchKernelGGL(rdf_kernel, dim3(grid), dim3(256), sizeof(unsigned int) * static_cast<size_t>(nbins), stream_,
-                           h.pos, h.meta, h.n, type_a, type_b, h.L, h.half, 1.0 / dr, nbins, d_counts);
+        const int tiles = (nb + 255) / 256;
+        // about 2048 blocks, each with at least 32 i for its histogram's clear and flush
+        const int runs = std::max(1, std::min((h.n + 31) / 32, 2048 / tiles));
+        const int len = (h.n + runs - 1) / runs;
+        const double edge = static_cast<double>(nbins) * dr;
+        hipLaunchKernelGGL(rdf_kernel, dim3(static_cast<unsigned>(tiles), static_cast<unsigned>((h.n + len - 1) / len)),
+                           dim3(256), sizeof(unsigned int) * static_cast<size_t>(nbins), stream_, h.pos, h.meta, h.n, type_a,
+                           type_b, h.L, h.half, 1.0 / dr, edge * edge * (1.0 + 1e-9), nbins, len,
+                           reinterpret_cast<const int*>(d), nb, d_counts);
         check_hip(hipGetLastError(), "rdf_kernel launch");
         check_hip(hipMemcpyAsync(part.data(), d_counts, sizeof(unsigned long long) * static_cast<size_t>(nbins),
                                  hipMemcpyDeviceToHost, stream_),
                   "copy rdf");
         check_hip(hipStreamSynchronize(stream_), "rdf sync");
     } catch (...) {
-        (void)hipFree(d_counts);
+        (void)hipStreamSynchronize(stream_);
+        (void)hipFree(d);
         throw;
     }
-    check_hip(hipFree(d_counts), "hipFree rdf");
+    check_hip(hipFree(d), "hipFree rdf");
     for (int b = 0; b < nbins; ++b) counts[b] += part[static_cast<size_t>(b)];
 }
 

@@ -1,7 +1,7 @@
 """Full recomputes at the sizes where their tiling can go wrong: Q(k) (whole and broken
 particle chunks, one and several column and nz blocks, a k list without its centre column's
 neighbours, a box with three lengths) and all pairs (tile edges, short runs, with and without
-a cutoff) against the oracle."""
+a cutoff) against the oracle; the pair-distance histogram across tile edges against numpy."""
 import numpy as np
 import pytest
 
@@ -38,3 +38,20 @@ def test_full_energy(n, kmax, box, cut):
     orc, eng, e_cpu, e_gpu = build_pair(ions(n, kmax, box, cut), F.Engine)
     assert abs(e_gpu - e_cpu) <= 1e-10 * max(1.0, abs(e_cpu))
     np.testing.assert_allclose(eng.total_energy()[1], orc.total_energy()[1], rtol=1e-10, atol=1e-10)
+
+
+@pytest.mark.parametrize("n,a,b,nbins", [(2, 0, 1, 7), (511, 0, 1, 300), (513, 1, 1, 64), (1200, 0, 0, 5)])
+def test_rdf_tiles(n, a, b, nbins):
+    cfg, xyz, q, ids, g = ions(n, 3, cut=12.0)
+    batch = F.Batch()
+    batch.add((cfg, xyz, q, ids, g), seed=1)
+    dr = 0.11
+    d = xyz[ids == a][:, None] - xyz[ids == b][None]
+    d = np.where(d > 30.0, d - 60.0, np.where(d < -30.0, d + 60.0, d))
+    r = np.sqrt((d[..., 0] * d[..., 0] + d[..., 1] * d[..., 1]) + d[..., 2] * d[..., 2])
+    if a == b:
+        r = r[np.triu_indices(len(r), 1)]
+    k = np.floor(r * (1.0 / dr)).ravel()
+    counts = np.bincount(k[k < nbins].astype(int), minlength=nbins).astype(np.uint64)
+    np.testing.assert_array_equal(batch.rdf(0, a, b, dr, nbins), counts)
+    batch.close()
