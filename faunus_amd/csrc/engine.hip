@@ -240,10 +240,7 @@ __global__ __launch_bounds__(kBlock) void delta_kernel(
                 const int a = e / (6 * width);
                 const double4 P = st == 0 ? mp[a].newp : mp[a].oldp;
                 const double x = axis == 0 ? P.x : (axis == 1 ? P.y : P.z);
-                const double kk = twopi * (static_cast<double>(nn) / box.L[axis]);
-                double sn, cs;
-                sincos(kk * x, &sn, &cs);
-                s_phase[e] = make_double2(cs, sn);
+                s_phase[e] = axis_phase(nn, x, 1.0 / box.L[axis]);
             }
             __syncthreads();
             for (int k = eb * kBlock + tid; k < nk; k += e_blocks * kBlock) {
@@ -408,7 +405,7 @@ __global__ __launch_bounds__(kQThreads) void full_q_kernel(const double4* __rest
     extern __shared__ double2 s_tab[]; // [chunk][3][ncut + 1], the x table times the charge
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int w = ncut + 1, row = 3 * w;
-    const double twopi = 6.283185307179586;
+    const double inv[3] = {1.0 / box.L[0], 1.0 / box.L[1], 1.0 / box.L[2]};
     const int c0 = kQTiles * 16 * static_cast<int>(blockIdx.z); // first (cos, sin) x nz entry of this block
     int nx[kCT], ny[kCT], tiles[kCT];
     double sy[kCT];
@@ -436,9 +433,8 @@ __global__ __launch_bounds__(kQThreads) void full_q_kernel(const double4* __rest
             if (base + j < j1) {
                 const double4 p = pos[base + j];
                 const double x = axis == 0 ? p.x : (axis == 1 ? p.y : p.z);
-                double sn, cs;
-                sincos(twopi * (static_cast<double>(r - axis * w) / box.L[axis]) * x, &sn, &cs);
-                v = axis == 0 ? make_double2(p.w * cs, p.w * sn) : make_double2(cs, sn);
+                v = axis_phase(r - axis * w, x, inv[axis]);
+                if (axis == 0) v = make_double2(p.w * v.x, p.w * v.y);
             }
             s_tab[e] = v;
         }
@@ -710,6 +706,7 @@ void Engine::upload_potentials() {
                 T.rmax2 = s.rmax2;
                 T.n = n;
                 T.hs = s.hardsphere ? 1 : 0;
+                std::fill(T.knots, T.knots + 2 * kSplMaxKnots, s.table.knots.back());
                 std::copy(s.table.knots.begin(), s.table.knots.end(), T.knots);
                 std::copy(s.table.coeff.begin(), s.table.coeff.end(), T.coeff);
                 T.x0 = s.table.knots.front();
@@ -743,6 +740,7 @@ void Engine::upload_potentials() {
     if (c.splined && (c.scheme == kCoulEwald || c.scheme == kCoulFanourgakis)) {
         if (static_cast<int>(c.S.knots.size()) > kMaxKnots) throw std::runtime_error("spline has too many knots");
         h_coul_.nknots = static_cast<int>(c.S.knots.size());
+        std::fill(h_coul_.knots, h_coul_.knots + kMaxKnots + 4, c.S.knots.back());
         std::copy(c.S.knots.begin(), c.S.knots.end(), h_coul_.knots);
         std::copy(c.S.coeff.begin(), c.S.coeff.end(), h_coul_.coeff);
         for (int b = 0; b <= kSplineBuckets; ++b) {
@@ -1065,6 +1063,38 @@ double Engine::interaction_range() const {
     for (double v : model_.g2g2) c2 = std::max(c2, v);
     // 1e-6 A above the bound: rigid rotations keep the atom distances up to rounding
     return std::min(range, std::sqrt(c2) + 2.0 * rmax + 1e-6);
+}
+
+bool Engine::rigid_reach(double* reach, double* sure) const {
+    if (g_begin_.empty()) return false;
+    double rmax = 0.0, cmin = kInf, cmax = 0.0;
+    for (size_t g = 0; g < g_begin_.size(); ++g) {
+        const MoleculeCfg& mol = model_.molecules[static_cast<size_t>(g_molid_[g])];
+        if (mol.atomic || !mol.rigid) return false;
+        for (int k = 0; k < g_size_[g]; ++k) {
+            const int i = g_begin_[g] + k;
+            double r2 = 0.0;
+            for (int d = 0; d < 3; ++d) {
+                double x = h_xyz_[3 * static_cast<size_t>(i) + d] - g_cm_[3 * g + d];
+                x -= model_.box[d] * std::round(x / model_.box[d]);
+                r2 += x * x;
+            }
+            rmax = std::max(rmax, std::sqrt(r2));
+        }
+    }
+    for (double v : model_.g2g2) {
+        cmin = std::min(cmin, std::sqrt(v));
+        cmax = std::max(cmax, std::sqrt(v));
+    }
+    // 1e-5 A for rounding of rotated atoms; 5e-6 of the cutoff for 32-bit centre distances
+    *reach = model_.pair_range + 2.0 * rmax + 1e-5;
+    *reach *= 1.0 + 1e-6;
+    *sure = kInf;
+    if (model_.has_g2g()) {
+        *reach = std::min(*reach, cmax * (1.0 + 5e-6));
+        *sure = cmin * (1.0 - 5e-6);
+    }
+    return std::isfinite(*reach);
 }
 
 void Engine::build_cell_list() {

@@ -21,7 +21,7 @@ constexpr int kPhaseTableMoved = 8;    // moved particles with LDS phase tables 
 constexpr int kBlock = 256;
 constexpr int kSplMaxKnots = 24;   // knots of one nonbonded_splined table (utol 1e-3 gives 7-10)
 constexpr int kSplMaxTables = 10;  // distinct type pairs with a table (four atom types)
-constexpr int kSplBuckets = 32;    // uniform buckets in r^2 indexing a table's knots
+constexpr int kSplBuckets = 256;   // uniform buckets in r^2 indexing a table's knots
 
 // Device copy of one type pair's parameters (64 bytes).
 struct DevPair {
@@ -34,12 +34,12 @@ struct DevPair {
 // One nonbonded_splined table (SplinedPotential's KnotData, potentials.h:773-781): the
 // Andrea spline of the exact pair energy in r^2 on [rmin2, rmax2]; bucket[b] is the first
 // knot >= x0 + b / inv_w, where the interval search starts.
-struct DevSplineTable {
+struct alignas(16) DevSplineTable {
     double rmin2, rmax2, x0, inv_w;
     int n, steps, hs, pad;
-    double knots[kSplMaxKnots];
     double coeff[6 * kSplMaxKnots];
-    unsigned char bucket[kSplBuckets + 8];
+    double knots[2 * kSplMaxKnots]; // padded with the last one past the search window
+    unsigned char bucket[kSplBuckets + 16];
 };
 
 // Device copy of the nonbonded model's shared data: the Coulomb scheme, its constants
@@ -50,8 +50,8 @@ struct alignas(16) DevCoulomb {
     int nknots;
     int spline_steps; // forward steps from a bucket's start that always reach the interval
     double lB, rc, rc_inv, alpha;
-    double knots[kMaxKnots];
     double coeff[6 * kMaxKnots];
+    double knots[kMaxKnots + 4]; // padded with the last one past the search window
     // bucket[b]: index of the first knot >= b / kSplineBuckets (start of the interval search)
     unsigned short bucket[kSplineBuckets + 1];
     int nspl;
@@ -164,6 +164,13 @@ class Engine {
     // cell, 4 x the mean + 32); a fixed capacity must hold the fullest initial cell.
     void set_cell_capacity(int cap);
     int cell_capacity() const { return cells_.cap; }
+    // Whether the caller fixed the members per cell of the current cell list.
+    bool cell_capacity_fixed() const { return cell_capacity_ > 0; }
+    // A system made only of rigid molecules: distances of two mass centres from which
+    // (reach) no pair of their atoms interacts, and below which (sure) the group cutoff
+    // surely does not cut them (infinite without one).  False when there is no such reach.
+    bool rigid_reach(double* reach, double* sure) const;
+    int num_columns() const { return ncol_; }
 
     // Pair-parameter and spline tables (as uploaded).
     const std::vector<DevPair>& dev_pairs() const { return h_pairs_; }

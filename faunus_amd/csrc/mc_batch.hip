@@ -150,10 +150,7 @@ __global__ __launch_bounds__(kThreads) void mc_advance_kernel(ReplicaState* __re
             const int st = e / (3 * width);
             const double x = st == 0 ? (axis == 0 ? nx_ : (axis == 1 ? ny_ : nz_))
                                      : (axis == 0 ? po.x : (axis == 1 ? po.y : po.z));
-            const double kk = 6.283185307179586 * (static_cast<double>(nn) / L);
-            double sn, cs;
-            sincos(kk * x, &sn, &cs);
-            s_phase[e] = make_double2(cs, sn);
+            s_phase[e] = axis_phase(nn, x, inv);
         }
 
         // nonbonded pair sums of the moved particle in the new and old position

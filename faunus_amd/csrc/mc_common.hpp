@@ -120,7 +120,14 @@ constexpr double kFixInv = 2.3283064365386963e-10; // 2^-32
 // round(x 2^32 / L) + 2^31 modulo 2^32 for x in [-L/2, L/2]; `s` = 2^32 / L.  One
 // multiply and a round to nearest even: the same word on the host and the device.
 __host__ __device__ inline uint32_t fixed_coord(double x, double s) {
+#ifdef __HIP_DEVICE_COMPILE__
+    // adding 1.5 x 2^52 rounds to the nearest integer and leaves it, modulo 2^32, in the low
+    // word (no 64-bit conversion); the product is rounded first, as on the host
+    const double v = __dadd_rn(__dmul_rn(x, s), 6755399441055744.0);
+    return static_cast<uint32_t>(__double_as_longlong(v)) + 0x80000000u;
+#else
     return static_cast<uint32_t>(static_cast<long long>(rint(x * s)) + 2147483648ll);
+#endif
 }
 
 __host__ __device__ inline FixPos fixed_pos(double x, double y, double z, double q, double inv) {
@@ -375,6 +382,16 @@ __device__ __forceinline__ bool metropolis(double du, double u) {
     return u <= exp(-du);
 }
 
+
+// metropolis with -log(u) at hand: decided against it away from the boundary (the margin
+// exceeds the rounding of exp and log many times), by exp itself only within the margin, so
+// the decision is the same without exp on the chain.
+__device__ __forceinline__ bool metropolis_log(double du, double u, double neg_log_u) {
+    const double margin = 1e-12 * (1.0 + fabs(neg_log_u));
+    if (du < neg_log_u - margin) return true;
+    if (du > neg_log_u + margin) return false;
+    return metropolis(du, u);
+}
 
 // Exclusive prefix sum of one int per thread over a block of kThreads threads
 // (wavefront shuffles, then the wave totals in LDS); *total receives the block sum.

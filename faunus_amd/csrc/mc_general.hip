@@ -932,9 +932,7 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
                 const int a = e / (6 * width);
                 const double4 A = st == 0 ? s_new[cst + a] : s_old[cst + a];
                 const double x = axis == 0 ? A.x : (axis == 1 ? A.y : A.z);
-                double sn, cs;
-                sincos(6.283185307179586 * (static_cast<double>(nn) / L) * x, &sn, &cs);
-                s_phase[e] = make_double2(cs, sn);
+                s_phase[e] = axis_phase(nn, x, inv);
             }
             __syncthreads();
 #pragma unroll

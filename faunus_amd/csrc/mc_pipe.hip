@@ -295,9 +295,7 @@ __global__ __launch_bounds__(256) void mc_pipe_kernel(ReplicaState* __restrict__
             const int st = e / (3 * width);
             const double x = st == 0 ? (axis == 0 ? nx_ : (axis == 1 ? ny_ : nz_))
                                      : (axis == 0 ? po.x : (axis == 1 ? po.y : po.z));
-            double sn, cs;
-            sincos((6.283185307179586 * (static_cast<double>(nn) / L)) * x, &sn, &cs);
-            s_phase[e] = make_double2(cs, sn);
+            s_phase[e] = axis_phase(nn, x, inv);
         }
         // pair sums (workgroup 0): committed configuration without i and the pending particles
         double acc_a = 0.0, acc_pn = 0.0, acc_po = 0.0;

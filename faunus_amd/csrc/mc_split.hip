@@ -254,9 +254,7 @@ __device__ __attribute__((always_inline)) inline void split_body(SplitLds<kThrea
             const int axis = (e / width) % 3;
             const int st = e / (3 * width);
             const double x = st == 0 ? (axis == 0 ? px : (axis == 1 ? py : pz)) : (axis == 0 ? ox : (axis == 1 ? oy : oz));
-            double sn, cs;
-            sincos((6.283185307179586 * (static_cast<double>(nn) / L)) * x, &sn, &cs);
-            s_phase[e] = make_double2(cs, sn);
+            s_phase[e] = axis_phase(nn, x, inv);
         }
     };
     // dQ of the move whose phase tables are in LDS (charge w), into dq1, and the thread's
