@@ -839,6 +839,7 @@ ReplicaState make_replica_state(Engine& e, bool fp32, unsigned long long seed, i
         std::vector<double> mw(static_cast<size_t>(m.ntypes));
         for (int t = 0; t < m.ntypes; ++t) mw[static_cast<size_t>(t)] = m.atoms[static_cast<size_t>(t)].mw;
         s.mw = upload(mw, owned, "upload atom masses");
+        set_rigid_fields(e, s, *kinds);
     }
     std::vector<double> terms(static_cast<size_t>(e.num_terms()));
     e.total_energy(terms.data());
@@ -910,6 +911,7 @@ int Batch::add_replica(const std::string& config_json, int n, const double* xyz,
                                         kinds);
     general_ = general;
     h_states_.push_back(s);
+    kinds_.push_back(kinds ? *kinds : std::vector<MoveKindSpec>());
     engines_.push_back(std::move(e));
     return s.replica_id;
 }
@@ -1138,6 +1140,11 @@ void Batch::set_replica_state(int r, const double* xyz, const double* mass_cente
             s->cell_members = cl.members;
             s->cell_of = cl.cell_of;
         }
+    }
+    const auto& kinds = kinds_[static_cast<size_t>(r)];
+    if (!kinds.empty()) {
+        set_rigid_fields(e, cur, kinds);
+        set_rigid_fields(e, h, kinds);
     }
     if (cur.surf != 0.0) {
         replica_dipole(e, cur.dip);

@@ -98,6 +98,11 @@ struct ReplicaState {
     double dip[3];            // surface term: the replica's dipole sum q r (positions as stored)
     double surf;              // surface term prefactor const_inf 2 pi lB / ((2 eps_s + 1) V), 0 without it
     int cell_radius;          // stencil half-width in cells (1: 27 cells, 2: 125 cells)
+    // rigid molecules only (mc_rigid_kernel): 0, or the largest group; molecules whose centres
+    // are at least sqrt(reach2) apart do not interact, those closer than sqrt(sure2) are not cut
+    int rigid, ngroups;
+    int rigid_even;           // every group has `rigid` atoms
+    double reach2, sure2;
     int threads;              // workgroup size of the translate-only kernel chosen by the tuner (0: the default rule)
 };
 
@@ -151,6 +156,14 @@ void launch_advance(const ReplicaState* h_states, int count, ReplicaState* d_sta
 void launch_general(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
                     TraceEntry* trace, int trace_cap, hipStream_t stream, const int2* d_blockmap = nullptr,
                     int map_blocks = 0);
+// Replicas in which every group is a small rigid molecule moved by translate+rotate
+// (mc_rigid_kernel): whether a replica takes that route when it is not shared by several
+// workgroups, a function of the replica alone, and the launch of `count` such replicas.
+bool rigid_route(const ReplicaState& s, bool f32);
+void launch_rigid(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
+                  TraceEntry* trace, int trace_cap, hipStream_t stream);
+// Fill a replica's fields for that route from its engine (after init or reset_positions).
+void set_rigid_fields(const Engine& e, ReplicaState& s, const std::vector<MoveKindSpec>& kinds);
 // Share a replica among `parts` workgroups of later general launches (1 undoes it);
 // allocates its exchange slots into `owned`.
 void set_replica_parts(ReplicaState& s, int parts, std::vector<void*>& owned);
@@ -247,6 +260,7 @@ class Batch {
     int cell_divisions_ = 1;
     int cell_capacity_ = 0;
     std::vector<std::unique_ptr<Engine>> engines_;
+    std::vector<std::vector<MoveKindSpec>> kinds_; // per replica (empty: translate only)
     std::vector<ReplicaState> h_states_;
     std::vector<void*> owned_; // device buffers made for the replicas
     ReplicaState* d_states_ = nullptr;
