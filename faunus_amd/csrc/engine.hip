@@ -5,7 +5,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
+#include <cstddef>
 #include <cstring>
 #include <numeric>
 #include <stdexcept>
@@ -45,28 +47,64 @@ __device__ __forceinline__ int cell_coord(double x, double half, double inv_cell
     return c;
 }
 
+// The DevCoulomb header and the `nspl` tables in use, by all threads of the block (the whole
+// struct is 22 KB, a system without tables needs 6).
+__device__ __forceinline__ void copy_coulomb(DevCoulomb& dst, const DevCoulomb* __restrict__ src, int nspl, int tid,
+                                             int nthreads) {
+    static_assert(offsetof(DevCoulomb, spl) % 16 == 0 && sizeof(DevSplineTable) % 16 == 0, "16-byte granules");
+    const uint4* s = reinterpret_cast<const uint4*>(src);
+    uint4* d = reinterpret_cast<uint4*>(&dst);
+    const int words = static_cast<int>((offsetof(DevCoulomb, spl) + static_cast<size_t>(nspl) * sizeof(DevSplineTable)) / 16);
+    for (int i = tid; i < words; i += nthreads) d[i] = s[i];
+}
+
+// Position of particle j in the moved set (sorted by index), or -1.
+__device__ __forceinline__ int moved_slot(const MovedParticle* mp, int m, int j) {
+    int lo = 0, hi = m;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (mp[mid].idx < j) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo < m && mp[lo].idx == j ? lo : -1;
+}
+
+// How the pair blocks of delta_kernel share the work: without a cell list, block b takes
+// every j_blocks-th run of 256 particles from run b mod j_blocks on, against the b div
+// j_blocks-th run of a_run moved atoms; with one, `lanes` lanes walk each (moved atom,
+// state, cell).  The Ewald blocks build phase tables of `chunk` moved particles at a time.
+struct PairSplit {
+    int blocks, j_blocks, a_run, lanes, nspl, chunk;
+};
+
 // ------------------------------------------------------------------------------
-// Fused per-move kernel.  Blocks [0, pair_blocks) sum the pair energies of the
-// affected pairs in the new and old state; blocks [pair_blocks, grid) update the
+// Fused per-move kernel.  Blocks [0, split.blocks) sum the pair energies of the
+// affected pairs in the new and old state; blocks [split.blocks, ewald_end) update the
 // trial structure factors Q_trial(k) = Q_acc(k) + dQ(k) and sum A_k|Q|^2 for both
 // states.  The last block to finish reduces all block partials in a fixed order
 // and writes the results to host-visible memory.
+// A launch is a few microseconds of latencies, so the kernel avoids what waits: partials and
+// results travel as agent- and system-scope stores completed by a wait (a fence would write
+// back the L2 of each block's XCD), the last block reads all partials at once (one thread
+// read them one after the other: 88 of them at K = 17328), and the pairs are spread over as
+// many lanes as there are.  Kernel time before -> now: 200 ions (cell list of 27 cells) 18.2 -> 8.8 us,
+// 20000 Na/Cl 23.6 -> 8.3 us, 1000 waters with a group cutoff 43.9 -> 13.5 us.
 // ------------------------------------------------------------------------------
 template <bool kGroups, bool kCells>
 __global__ __launch_bounds__(kBlock) void delta_kernel(
     const double4* __restrict__ pos, const uint32_t* __restrict__ meta, int n, const DevPair* __restrict__ pairs_g,
     int ntypes, const DevCoulomb* __restrict__ coul_g, Box box, GroupTable groups, CellArgs cells, MoveArgs mv,
-    int pair_blocks, const int* __restrict__ kn, const double* __restrict__ ak, const double2* __restrict__ q_acc,
-    double2* __restrict__ q_trial, int nk, int ncut, double2* __restrict__ partials, unsigned* __restrict__ ticket,
+    PairSplit split, const int* __restrict__ kn, const double* __restrict__ ak, const double2* __restrict__ q_acc,
+    double2* __restrict__ q_trial, int nk, int ncut, double* __restrict__ partials, unsigned* __restrict__ ticket,
     DeltaResult* __restrict__ out, unsigned long long seq, double rec_prefactor, double cm_new_x, double cm_new_y,
     double cm_new_z, double cm_old_x, double cm_old_y, double cm_old_z, int ewald_end,
     const int* __restrict__ bond_off, const DevBond* __restrict__ bonds) {
     __shared__ DevPair s_pairs[kMaxTypes * kMaxTypes];
     __shared__ DevCoulomb s_coul;
     __shared__ MovedParticle s_moved[kPhaseTableMoved];
-    __shared__ double s_red[2][kBlock / 64];
+    __shared__ double s_red[6][kBlock / 64];
     __shared__ bool s_last;
-    extern __shared__ double2 s_phase[]; // Ewald phase tables
+    extern __shared__ double2 s_phase[]; // Ewald phase tables of up to kPhaseTableMoved moved particles
 
     const int tid = threadIdx.x;
     const int m = mv.m;
@@ -76,14 +114,15 @@ __global__ __launch_bounds__(kBlock) void delta_kernel(
     const MovedParticle* mp = (m <= kPhaseTableMoved) ? s_moved : moved;
 
     double acc_new = 0.0, acc_old = 0.0;
-    const bool is_pair_block = static_cast<int>(blockIdx.x) < pair_blocks;
+    const bool is_pair_block = static_cast<int>(blockIdx.x) < split.blocks;
     if (is_pair_block) {
         for (int i = tid; i < ntypes * ntypes; i += kBlock) s_pairs[i] = pairs_g[i];
-        lds_copy(s_coul, coul_g, tid, kBlock);
+        copy_coulomb(s_coul, coul_g, split.nspl, tid, kBlock);
         __syncthreads();
         const bool single = mv.change_group >= 0;
-        auto allowed_other = [&](int gi, int gj, bool new_state) -> bool {
-            // pair between a moved particle in group gi and a static particle in group gj
+        // pair of a moved particle in group gi (the changed group when there is one) with a
+        // static particle in group gj
+        auto allowed = [&](int gi, int gj, bool new_state) -> bool {
             if (gi == gj) return single && mv.internal && (!kGroups || !(groups.flags[gi] & 2));
             if (!kGroups) return true;
             if (groups.g2g2 && (groups.flags[gi] & 1) && (groups.flags[gj] & 1)) { // GroupCutoff::cut (energy.h:761-768)
@@ -94,58 +133,51 @@ __global__ __launch_bounds__(kBlock) void delta_kernel(
             }
             return true;
         };
-        auto visit = [&](int j, const double4 pj, uint32_t mj) {
-            const int tj = static_cast<int>(mj & 0xffu);
-            const int gj = static_cast<int>(mj >> 8);
-            // is j one of the moved particles (sorted by index)?
-            int jm = -1;
-            {
-                int lo = 0, hi = m;
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (mp[mid].idx < j) lo = mid + 1;
-                    else hi = mid;
+        // pair of two moved particles, each at its state's coordinates
+        auto moved_pair = [&](const MovedParticle& A, const MovedParticle& B) {
+            // several moved groups are atomic (molecular multi-group changes are rejected on the host)
+            const bool ok = A.gid != B.gid || (single && mv.internal &&
+                                               (!kGroups || (!(groups.flags[A.gid] & 2) &&
+                                                             !pair_excluded(groups.excl_off, groups.excl, A.idx, B.idx))));
+            if (!ok) return;
+            const DevPair& p = s_pairs[A.type * ntypes + B.type];
+            acc_new += pair_energy(p, s_coul, A.newp.w, B.newp.w,
+                                   dist2(box, A.newp.x, A.newp.y, A.newp.z, B.newp.x, B.newp.y, B.newp.z));
+            acc_old += pair_energy(p, s_coul, A.oldp.w, B.oldp.w,
+                                   dist2(box, A.oldp.x, A.oldp.y, A.oldp.z, B.oldp.x, B.oldp.y, B.oldp.z));
+        };
+        if (!kCells) {
+            const int a0 = static_cast<int>(blockIdx.x) / split.j_blocks * split.a_run, a1 = min(m, a0 + split.a_run);
+            for (int j = (static_cast<int>(blockIdx.x) % split.j_blocks) * kBlock + tid; j < n; j += split.j_blocks * kBlock) {
+                const double4 pj = pos[j];
+                const uint32_t mj = meta[j];
+                const int tj = static_cast<int>(mj & 0xffu), gj = static_cast<int>(mj >> 8);
+                const int jm = moved_slot(mp, m, j);
+                if (jm >= 0) {
+                    for (int a = a0; a < min(a1, jm); ++a) moved_pair(mp[a], mp[jm]);
+                    continue;
                 }
-                if (lo < m && mp[lo].idx == j) jm = lo;
-            }
-            if (jm < 0) {
-                for (int a = 0; a < m; ++a) {
+                const bool ok_new = !single || allowed(mv.change_group, gj, true);
+                const bool ok_old = !single || allowed(mv.change_group, gj, false);
+                if (!ok_new && !ok_old) continue;
+                for (int a = a0; a < a1; ++a) {
                     const MovedParticle& M = mp[a];
+                    if (!single && M.gid == gj) continue;
                     if (kGroups && M.gid == gj && pair_excluded(groups.excl_off, groups.excl, M.idx, j)) continue;
                     const DevPair& p = s_pairs[M.type * ntypes + tj];
-                    if (allowed_other(M.gid, gj, true))
+                    if (ok_new)
                         acc_new += pair_energy(p, s_coul, M.newp.w, pj.w,
                                                dist2(box, M.newp.x, M.newp.y, M.newp.z, pj.x, pj.y, pj.z));
-                    if (allowed_other(M.gid, gj, false))
+                    if (ok_old)
                         acc_old += pair_energy(p, s_coul, M.oldp.w, pj.w,
                                                dist2(box, M.oldp.x, M.oldp.y, M.oldp.z, pj.x, pj.y, pj.z));
                 }
-            } else {
-                // moved <-> moved pairs (a < jm), both particles at their state's coordinates
-                const MovedParticle& B = mp[jm];
-                for (int a = 0; a < jm; ++a) {
-                    const MovedParticle& A = mp[a];
-                    bool ok;
-                    if (A.gid == B.gid)
-                        ok = single && mv.internal && (!kGroups || (!(groups.flags[A.gid] & 2) &&
-                                                                    !pair_excluded(groups.excl_off, groups.excl, A.idx, B.idx)));
-                    else ok = true; // several moved groups: atomic (molecular multi-group changes are rejected on the host)
-                    if (!ok) continue;
-                    const DevPair& p = s_pairs[A.type * ntypes + B.type];
-                    acc_new += pair_energy(p, s_coul, A.newp.w, B.newp.w,
-                                           dist2(box, A.newp.x, A.newp.y, A.newp.z, B.newp.x, B.newp.y, B.newp.z));
-                    acc_old += pair_energy(p, s_coul, A.oldp.w, B.oldp.w,
-                                           dist2(box, A.oldp.x, A.oldp.y, A.oldp.z, B.oldp.x, B.oldp.y, B.oldp.z));
-                }
             }
-        };
-        if (!kCells) {
-            for (int j = blockIdx.x * kBlock + tid; j < n; j += pair_blocks * kBlock) visit(j, pos[j], meta[j]);
         } else {
             // Stencils of 27 cells around each moved particle's new and old position;
             // candidates are evaluated only for the state whose stencil holds them.
-            const int stencil_jobs = m * 2 * 27;
-            for (int job = blockIdx.x; job < stencil_jobs; job += pair_blocks) {
+            const int first = (static_cast<int>(blockIdx.x) * kBlock + tid) / split.lanes;
+            for (int job = first; job < m * 54; job += split.blocks * kBlock / split.lanes) {
                 const int a = job / 54;
                 const int s = (job / 27) & 1; // 0: new, 1: old
                 const int c = job % 27;
@@ -156,17 +188,14 @@ __global__ __launch_bounds__(kBlock) void delta_kernel(
                 const int cz = (cell_coord(P.z, box.half[2], cells.inv2, cells.nc2) + (c / 9) - 1 + cells.nc2) % cells.nc2;
                 const int cell = (cz * cells.nc1 + cy) * cells.nc0 + cx;
                 const int cnt = cells.count[cell];
-                for (int k = tid; k < cnt; k += kBlock) {
+                for (int k = tid & (split.lanes - 1); k < cnt; k += split.lanes) {
                     const int j = cells.members[cell * cells.cap + k];
                     const double4 pj = pos[j];
                     const uint32_t mj = meta[j];
-                    int jm = -1;
-                    for (int b = 0; b < m; ++b)
-                        if (mp[b].idx == j) jm = b;
-                    if (jm >= 0) continue; // moved <-> moved handled below
+                    if (moved_slot(mp, m, j) >= 0) continue; // moved <-> moved handled below
                     const int tj = static_cast<int>(mj & 0xffu);
                     const int gj = static_cast<int>(mj >> 8);
-                    if (!allowed_other(M.gid, gj, s == 0)) continue;
+                    if (!allowed(M.gid, gj, s == 0)) continue;
                     if (kGroups && M.gid == gj && pair_excluded(groups.excl_off, groups.excl, M.idx, j)) continue;
                     const DevPair& p = s_pairs[M.type * ntypes + tj];
                     const double u = pair_energy(p, s_coul, P.w, pj.w, dist2(box, P.x, P.y, P.z, pj.x, pj.y, pj.z));
@@ -174,25 +203,11 @@ __global__ __launch_bounds__(kBlock) void delta_kernel(
                     else acc_old += u;
                 }
             }
-            if (blockIdx.x == 0) {
+            if (blockIdx.x == 0)
                 for (int pairidx = tid; pairidx < m * m; pairidx += kBlock) {
                     const int a = pairidx / m, b = pairidx % m;
-                    if (a >= b) continue;
-                    const MovedParticle& A = mp[a];
-                    const MovedParticle& B = mp[b];
-                    bool ok = (A.gid == B.gid)
-                                  ? (single && mv.internal &&
-                                     (!kGroups || (!(groups.flags[A.gid] & 2) &&
-                                                   !pair_excluded(groups.excl_off, groups.excl, A.idx, B.idx))))
-                                  : true;
-                    if (!ok) continue;
-                    const DevPair& p = s_pairs[A.type * ntypes + B.type];
-                    acc_new += pair_energy(p, s_coul, A.newp.w, B.newp.w,
-                                           dist2(box, A.newp.x, A.newp.y, A.newp.z, B.newp.x, B.newp.y, B.newp.z));
-                    acc_old += pair_energy(p, s_coul, A.oldp.w, B.oldp.w,
-                                           dist2(box, A.oldp.x, A.oldp.y, A.oldp.z, B.oldp.x, B.oldp.y, B.oldp.z));
+                    if (a < b) moved_pair(mp[a], mp[b]);
                 }
-            }
         }
     } else if (static_cast<int>(blockIdx.x) >= ewald_end) {
         // Bonded::internalGroupEnergy (energy.cpp:1068-1088): bonds with at least one
@@ -203,16 +218,7 @@ __global__ __launch_bounds__(kBlock) void delta_kernel(
                 const MovedParticle& A = mp[a];
                 for (int e = bond_off[A.idx]; e < bond_off[A.idx + 1]; ++e) {
                     const DevBond B = bonds[e];
-                    int om = -1;
-                    {
-                        int lo = 0, hi = m;
-                        while (lo < hi) {
-                            const int mid = (lo + hi) >> 1;
-                            if (mp[mid].idx < B.other) lo = mid + 1;
-                            else hi = mid;
-                        }
-                        if (lo < m && mp[lo].idx == B.other) om = lo;
-                    }
+                    const int om = moved_slot(mp, m, B.other);
                     if (om >= 0 && om < a) continue; // the pair is visited from the lower moved atom
                     const double4 on = om >= 0 ? mp[om].newp : pos[B.other];
                     const double4 oo = om >= 0 ? mp[om].oldp : on;
@@ -224,155 +230,159 @@ __global__ __launch_bounds__(kBlock) void delta_kernel(
             }
         }
     } else if (nk > 0) {
-        __syncthreads();
-        // Ewald partial update (energy.cpp:219-247): dQ(k) = sum_i q_i (e^{ik.r_new} - e^{ik.r_old}).
-        const int eb = blockIdx.x - pair_blocks;
-        const int e_blocks = ewald_end - pair_blocks;
+        // Ewald partial update (energy.cpp:219-247): dQ(k) = sum_i q_i (e^{ik.r_new} - e^{ik.r_old}),
+        // with e^{i k_a(n) r_a}, n in [-ncut, ncut], per moved particle, state and axis in
+        // LDS, split.chunk particles at a time; a thread holds two k-vectors
+        const int eb = static_cast<int>(blockIdx.x) - split.blocks;
+        const int e_blocks = ewald_end - split.blocks;
         const int width = 2 * ncut + 1;
-        const double twopi = 6.283185307179586;
-        if (m <= kPhaseTableMoved) {
-            // per moved particle, state and axis: e^{i k_a(n) r_a} for n in [-ncut, ncut]
-            const int entries = m * 2 * 3 * width;
-            for (int e = tid; e < entries; e += kBlock) {
-                const int nn = e % width - ncut;
-                const int axis = (e / width) % 3;
-                const int st = (e / (3 * width)) & 1;
-                const int a = e / (6 * width);
-                const double4 P = st == 0 ? mp[a].newp : mp[a].oldp;
-                const double x = axis == 0 ? P.x : (axis == 1 ? P.y : P.z);
-                s_phase[e] = axis_phase(nn, x, 1.0 / box.L[axis]);
+        for (int k0 = eb * 2 * kBlock; k0 < nk; k0 += e_blocks * 2 * kBlock) {
+            double dre[2] = {0.0, 0.0}, dim[2] = {0.0, 0.0};
+            int packed[2];
+            double2 qa[2];
+            double A[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int k = min(k0 + i * kBlock + tid, nk - 1);
+                packed[i] = kn[k];
+                qa[i] = q_acc[k];
+                A[i] = ak[k];
             }
-            __syncthreads();
-            for (int k = eb * kBlock + tid; k < nk; k += e_blocks * kBlock) {
-                const int packed = kn[k];
-                const int nx = unpack_n(packed, 0) + ncut, ny = unpack_n(packed, 1) + ncut,
-                          nz = unpack_n(packed, 2) + ncut;
-                double dre = 0.0, dim = 0.0;
-                for (int a = 0; a < m; ++a) {
-                    for (int st = 0; st < 2; ++st) {
-                        const double2* t = s_phase + (a * 2 + st) * 3 * width;
-                        const double2 ex = t[nx], ey = t[width + ny], ez = t[2 * width + nz];
-                        const double re1 = ex.x * ey.x - ex.y * ey.y;
-                        const double im1 = ex.x * ey.y + ex.y * ey.x;
-                        const double re = re1 * ez.x - im1 * ez.y;
-                        const double im = re1 * ez.y + im1 * ez.x;
-                        const double q = st == 0 ? mp[a].newp.w : -mp[a].oldp.w;
-                        dre += q * re;
-                        dim += q * im;
+            for (int c0 = 0; c0 < m; c0 += split.chunk) {
+                const int cm = min(split.chunk, m - c0);
+                __syncthreads(); // the moved particles, or the previous tables, are consumed
+                for (int e = tid; e < cm * 6 * width; e += kBlock) {
+                    const int nn = e % width - ncut;
+                    const int axis = (e / width) % 3;
+                    const int st = (e / (3 * width)) & 1;
+                    const MovedParticle& M = mp[c0 + e / (6 * width)];
+                    const double4 P = st == 0 ? M.newp : M.oldp;
+                    s_phase[e] = axis_phase(nn, axis == 0 ? P.x : (axis == 1 ? P.y : P.z), 1.0 / box.L[axis]);
+                }
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int nx = unpack_n(packed[i], 0) + ncut, ny = unpack_n(packed[i], 1) + ncut,
+                              nz = unpack_n(packed[i], 2) + ncut;
+                    for (int a = 0; a < cm; ++a) {
+#pragma unroll
+                        for (int st = 0; st < 2; ++st) {
+                            const double2* t = s_phase + (a * 2 + st) * 3 * width;
+                            const double2 ex = t[nx], ey = t[width + ny], ez = t[2 * width + nz];
+                            const double re1 = ex.x * ey.x - ex.y * ey.y;
+                            const double im1 = ex.x * ey.y + ex.y * ey.x;
+                            const double q = st == 0 ? mp[c0 + a].newp.w : -mp[c0 + a].oldp.w;
+                            dre[i] += q * (re1 * ez.x - im1 * ez.y);
+                            dim[i] += q * (re1 * ez.y + im1 * ez.x);
+                        }
                     }
                 }
-                const double2 qa = q_acc[k];
-                const double2 qt = make_double2(qa.x + dre, qa.y + dim);
-                q_trial[k] = qt;
-                const double A = ak[k];
-                acc_new += A * (qt.x * qt.x + qt.y * qt.y);
-                acc_old += A * (qa.x * qa.x + qa.y * qa.y);
             }
-        } else {
-            for (int k = eb * kBlock + tid; k < nk; k += e_blocks * kBlock) {
-                const int packed = kn[k];
-                const double kx = twopi * (static_cast<double>(unpack_n(packed, 0)) / box.L[0]);
-                const double ky = twopi * (static_cast<double>(unpack_n(packed, 1)) / box.L[1]);
-                const double kz = twopi * (static_cast<double>(unpack_n(packed, 2)) / box.L[2]);
-                double dre = 0.0, dim = 0.0;
-                for (int a = 0; a < m; ++a) {
-                    const MovedParticle& M = mp[a];
-                    double sn, cs;
-                    sincos(kx * M.newp.x + ky * M.newp.y + kz * M.newp.z, &sn, &cs);
-                    dre += M.newp.w * cs;
-                    dim += M.newp.w * sn;
-                    sincos(kx * M.oldp.x + ky * M.oldp.y + kz * M.oldp.z, &sn, &cs);
-                    dre -= M.oldp.w * cs;
-                    dim -= M.oldp.w * sn;
-                }
-                const double2 qa = q_acc[k];
-                const double2 qt = make_double2(qa.x + dre, qa.y + dim);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int k = k0 + i * kBlock + tid;
+                if (k >= nk) continue;
+                const double2 qt = make_double2(qa[i].x + dre[i], qa[i].y + dim[i]);
                 q_trial[k] = qt;
-                const double A = ak[k];
-                acc_new += A * (qt.x * qt.x + qt.y * qt.y);
-                acc_old += A * (qa.x * qa.x + qa.y * qa.y);
+                acc_new += A[i] * (qt.x * qt.x + qt.y * qt.y);
+                acc_old += A[i] * (qa[i].x * qa[i].x + qa[i].y * qa[i].y);
             }
         }
-    } else {
-        __syncthreads();
     }
 
-    // block partials
-    const double bn = block_sum<kBlock>(acc_new, s_red[0]);
-    const double bo = block_sum<kBlock>(acc_old, s_red[1]);
+    // block partials: stored at agent scope, complete before the block's ticket
+    const double bn = wave_sum(acc_new), bo = wave_sum(acc_old);
+    if ((tid & 63) == 0) {
+        s_red[0][tid >> 6] = bn;
+        s_red[1][tid >> 6] = bo;
+    }
+    __syncthreads();
     if (tid == 0) {
-        partials[blockIdx.x] = make_double2(bn, bo);
-        __threadfence();
-        const unsigned t = atomicAdd(ticket, 1u);
+        double v0 = 0.0, v1 = 0.0;
+        for (int w = 0; w < kBlock / 64; ++w) {
+            v0 += s_red[0][w];
+            v1 += s_red[1][w];
+        }
+        __hip_atomic_store(partials + 2 * blockIdx.x, v0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(partials + 2 * blockIdx.x + 1, v1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         s_last = (t == gridDim.x - 1);
     }
     __syncthreads();
     if (!s_last) return;
-    __threadfence();
-    // last block: fixed-order reduction of the pair partials and of the Ewald partials
-    double pn = 0.0, po = 0.0, en = 0.0, eo = 0.0, bn_ = 0.0, bo_ = 0.0;
-    if (tid == 0) {
-        for (int b = 0; b < static_cast<int>(gridDim.x); ++b) {
-            const double* pb = reinterpret_cast<const double*>(partials) + 2 * b;
-            const double2 v = make_double2(__hip_atomic_load(pb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-                                           __hip_atomic_load(pb + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            if (b < pair_blocks) {
-                pn += v.x;
-                po += v.y;
-            } else if (b < ewald_end) {
-                en += v.x;
-                eo += v.y;
-            } else {
-                bn_ += v.x;
-                bo_ += v.y;
-            }
+    // last block: fixed-order reduction of the pair, Ewald and bond partials
+    double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int b = tid; b < static_cast<int>(gridDim.x); b += kBlock) {
+        const double x = __hip_atomic_load(partials + 2 * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const double y = __hip_atomic_load(partials + 2 * b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int r = b < split.blocks ? 0 : (b < ewald_end ? 2 : 4);
+#pragma unroll
+        for (int k = 0; k < 6; k += 2) {
+            v[k] += r == k ? x : 0.0;
+            v[k + 1] += r == k ? y : 0.0;
         }
-        out->pair_new = pn;
-        out->pair_old = po;
-        out->rec_new = rec_prefactor * en;
-        out->rec_old = rec_prefactor * eo;
-        out->bond_new = bn_;
-        out->bond_old = bo_;
-        __threadfence_system();
-        out->seq = seq;
-        __threadfence_system();
-        *ticket = 0u;
+    }
+#pragma unroll
+    for (int r = 0; r < 6; ++r) {
+        const double x = wave_sum(v[r]);
+        if ((tid & 63) == 0) s_red[r][tid >> 6] = x;
+    }
+    __syncthreads();
+    if (tid < 6) {
+        double x = 0.0;
+        for (int w = 0; w < kBlock / 64; ++w) x += s_red[tid][w];
+        if (tid == 2 || tid == 3) x *= rec_prefactor;
+        // DeltaResult: pair, reciprocal and bond sums, each new and old
+        __hip_atomic_store(&out->pair_new + tid, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (tid == 0) {
+            *ticket = 0u;
+            __hip_atomic_store(&out->seq, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
 }
 
-// Accept: write the moved particles' trial coordinates into the accepted state and
-// move them between cells of the cell list (one thread, deterministic order).
-__global__ void commit_kernel(double4* pos, MoveArgs mv, CellArgs cells, int* cell_of, int* overflow, Box box,
-                              int use_cells) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// Accept: write the moved particles' trial coordinates into the accepted state, the moved
+// group's mass centre (cm_group >= 0) and move the particles between cells of the cell list
+// (one wave, in order; its lanes search a cell's members together).
+__global__ __launch_bounds__(64) void commit_kernel(double4* pos, MoveArgs mv, CellArgs cells, int* cell_of, int* overflow,
+                                                    Box box, int use_cells, double* gcm, int cm_group, double cx, double cy,
+                                                    double cz) {
+    const int lane = threadIdx.x;
     const MovedParticle* moved = (mv.m <= kMaxInlineMoved) ? mv.inl : mv.ext;
+    if (lane < 3 && cm_group >= 0) gcm[3 * cm_group + lane] = lane == 0 ? cx : (lane == 1 ? cy : cz);
+    for (int a = lane; a < mv.m; a += 64) pos[moved[a].idx] = moved[a].newp;
+    if (!use_cells) return;
+    int* cnt = const_cast<int*>(cells.count);
+    int* mem = const_cast<int*>(cells.members);
     for (int a = 0; a < mv.m; ++a) {
         const MovedParticle& M = moved[a];
-        pos[M.idx] = M.newp;
-        if (!use_cells) continue;
-        const int cx = cell_coord(M.newp.x, box.half[0], cells.inv0, cells.nc0);
-        const int cy = cell_coord(M.newp.y, box.half[1], cells.inv1, cells.nc1);
-        const int cz = cell_coord(M.newp.z, box.half[2], cells.inv2, cells.nc2);
-        const int cnew = (cz * cells.nc1 + cy) * cells.nc0 + cx;
+        const int x = cell_coord(M.newp.x, box.half[0], cells.inv0, cells.nc0);
+        const int y = cell_coord(M.newp.y, box.half[1], cells.inv1, cells.nc1);
+        const int z = cell_coord(M.newp.z, box.half[2], cells.inv2, cells.nc2);
+        const int cnew = (z * cells.nc1 + y) * cells.nc0 + x;
         const int cold = cell_of[M.idx];
         if (cnew == cold) continue;
-        int* cnt = const_cast<int*>(cells.count);
-        int* mem = const_cast<int*>(cells.members);
-        const int nold = cnt[cold];
-        for (int k = 0; k < nold; ++k)
-            if (mem[cold * cells.cap + k] == M.idx) {
-                mem[cold * cells.cap + k] = mem[cold * cells.cap + nold - 1];
-                break;
-            }
-        cnt[cold] = nold - 1;
-        const int nn = cnt[cnew];
-        if (nn >= cells.cap) {
-            *overflow = 1;
-            continue;
+        const int nold = cnt[cold], nn = cnt[cnew];
+        const int last = mem[cold * cells.cap + max(nold - 1, 0)];
+        int slot = -1;
+        for (int k = 0; k < nold && slot < 0; k += 64) {
+            const unsigned long long found = __ballot(k + lane < nold && mem[cold * cells.cap + min(k + lane, nold - 1)] == M.idx);
+            if (found) slot = k + __builtin_ctzll(found);
         }
-        mem[cnew * cells.cap + nn] = M.idx;
-        cnt[cnew] = nn + 1;
-        cell_of[M.idx] = cnew;
+        __syncthreads(); // every lane has read the lists
+        if (lane == 0) {
+            if (slot >= 0) mem[cold * cells.cap + slot] = last;
+            cnt[cold] = nold - 1;
+            if (nn >= cells.cap) *overflow = 1;
+            else {
+                mem[cnew * cells.cap + nn] = M.idx;
+                cnt[cnew] = nn + 1;
+                cell_of[M.idx] = cnew;
+            }
+        }
+        __syncthreads(); // the next particle sees the changed lists
     }
 }
 
@@ -1232,18 +1242,32 @@ void Engine::timing(double* total_ms, long* launches) {
     *launches = static_cast<long>(ev_pairs_.size());
 }
 
-void Engine::launch_delta(const MoveArgs& args, int pair_blocks, int ewald_blocks, bool bond_block) {
+void Engine::launch_delta(const MoveArgs& args, int ewald_blocks, bool bond_block) {
     const Box box = make_box(model_);
     GroupTable gt{d_gflags_, d_gcm_, d_g2g_, static_cast<int>(model_.molecules.size()), d_excl_off_, d_excl_};
     CellArgs ca{cells_.count, cells_.members, cells_.nc[0], cells_.nc[1], cells_.nc[2], cells_.cap,
                 cells_.inv_cell[0], cells_.inv_cell[1], cells_.inv_cell[2]};
-    const int ewald_end = pair_blocks + ewald_blocks;
+    const int ncut = model_.ewald.present ? static_cast<int>(std::ceil(model_.ewald.n_cutoff)) : 0;
+    PairSplit split{1, 1, args.m, kBlock, h_coul_.nspl, std::max(1, std::min(args.m, kPhaseTableMoved))};
+    const size_t table = sizeof(double2) * 6 * static_cast<size_t>(2 * ncut + 1); // one moved particle's
+    while (split.chunk > 1 && split.chunk * table > 16 * 1024) --split.chunk;
+    if (cells_.enabled) {
+        // as many lanes per cell as it holds particles on average (a power of two)
+        const double mean = static_cast<double>(n_) / (static_cast<double>(cells_.nc[0]) * cells_.nc[1] * cells_.nc[2]);
+        split.lanes = 4;
+        while (split.lanes < 64 && split.lanes < mean) split.lanes *= 2;
+        split.blocks = std::min((args.m * 54 * split.lanes + kBlock - 1) / kBlock, 256);
+    } else {
+        // one particle per thread, then runs of at least two moved atoms while CUs are free
+        split.j_blocks = std::max(1, std::min((n_ + kBlock - 1) / kBlock, 2 * num_cu_));
+        const int runs = std::max(1, std::min((args.m + 1) / 2, 2 * num_cu_ / split.j_blocks));
+        split.a_run = std::max(1, (args.m + runs - 1) / runs);
+        split.blocks = split.j_blocks * std::max(1, (args.m + split.a_run - 1) / split.a_run);
+    }
+    const int ewald_end = split.blocks + ewald_blocks;
     const int grid = ewald_end + (bond_block ? 1 : 0);
     if (grid > max_blocks_) throw std::runtime_error("too many blocks");
-    const int ncut = model_.ewald.present ? static_cast<int>(std::ceil(model_.ewald.n_cutoff)) : 0;
-    const size_t lds = (args.m <= kPhaseTableMoved && nk_ > 0)
-                           ? sizeof(double2) * static_cast<size_t>(args.m) * 2 * 3 * (2 * ncut + 1)
-                           : 0;
+    const size_t lds = nk_ > 0 ? static_cast<size_t>(split.chunk) * table : 0;
     const double V = model_.box[0] * model_.box[1] * model_.box[2];
     const double pref = model_.ewald.present ? 2 * kPi * model_.ewald.lB / V : 0.0;
     // reference order: 2*pi*energy*lB/V (energy.cpp:530); the prefactor is applied to
@@ -1271,8 +1295,8 @@ void Engine::launch_delta(const MoveArgs& args, int pair_blocks, int ewald_block
         throw std::runtime_error("the per-move path walks 27-cell stencils (cell divisions 1)");
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(kBlock), lds, stream_, d_pos_, d_meta_, n_, d_pairs_,
-                           model_.ntypes, d_coul_, box, gt, ca, args, pair_blocks, d_kn_, d_ak_, d_q_acc_, d_q_trial_,
-                           nk_, ncut, d_partials_, d_ticket_, h_result_, seq_, pref, cn[0], cn[1], cn[2], co[0], co[1],
+                           model_.ntypes, d_coul_, box, gt, ca, args, split, d_kn_, d_ak_, d_q_acc_, d_q_trial_,
+                           nk_, ncut, reinterpret_cast<double*>(d_partials_), d_ticket_, h_result_, seq_, pref, cn[0], cn[1], cn[2], co[0], co[1],
                            co[2], ewald_end, d_bond_off_, d_bond_);
     };
     if (any_molecular_) {
@@ -1288,6 +1312,20 @@ void Engine::launch_delta(const MoveArgs& args, int pair_blocks, int ewald_block
         ev_pairs_.emplace_back(e0, e1);
     }
     ++launches_;
+}
+
+// Wait for the result of launch seq_: the kernel's last block writes it to host memory with
+// the launch's number behind it, so the host need not wait for the end of the kernel and its
+// completion signal.  Work enqueued afterwards still follows the kernel on the stream.  A
+// result that does not come within 20 ms is left to the stream's synchronisation, which
+// reports a launch or device error.
+void Engine::wait_result() {
+    const auto start = std::chrono::steady_clock::now();
+    for (unsigned spins = 1; __atomic_load_n(&h_result_->seq, __ATOMIC_ACQUIRE) != seq_; ++spins) {
+        if ((spins & 0xfffu) != 0 || std::chrono::steady_clock::now() - start < std::chrono::milliseconds(20)) continue;
+        check_hip(hipStreamSynchronize(stream_), "delta sync");
+        return;
+    }
 }
 
 void Engine::delta(const std::vector<int>& groups, const std::vector<char>& all, const std::vector<char>& internal,
@@ -1348,18 +1386,15 @@ void Engine::delta(const std::vector<int>& groups, const std::vector<char>& all,
                   "copy moved");
         args.ext = d_moved_;
     }
-    int pair_blocks;
-    if (cells_.enabled) pair_blocks = std::min(args.m * 54, 256);
-    else pair_blocks = std::max(1, std::min((n_ + kBlock * 4 - 1) / (kBlock * 4), 2 * num_cu_));
     int ewald_blocks = 0;
     if (nk_ > 0) ewald_blocks = std::max(1, std::min((nk_ + 2 * kBlock - 1) / (2 * kBlock), 2 * num_cu_));
     if (single && any_molecular_ && model_.has_g2g() &&
         !model_.molecules[static_cast<size_t>(g_molid_[static_cast<size_t>(groups[0])])].atomic &&
         staged_cm_group_ != groups[0])
         throw std::runtime_error("delta: stage the trial mass centre of a moved molecular group when cutoff_g2g is set");
-    launch_delta(args, pair_blocks, ewald_blocks, nbonds_ > 0 && model_.bonded_term >= 0);
-    check_hip(hipStreamSynchronize(stream_), "delta sync");
-    volatile DeltaResult* r = h_result_;
+    launch_delta(args, ewald_blocks, nbonds_ > 0 && model_.bonded_term >= 0);
+    wait_result();
+    const DeltaResult* r = h_result_;
     if (r->seq != seq_) throw std::runtime_error("delta: result sequence mismatch");
     // dipole of the trial state (surface term, energy.cpp:466-482)
     for (int d = 0; d < 3; ++d) dipole_trial_[d] = dipole_[d];
@@ -1416,7 +1451,8 @@ void Engine::sync(bool accept) {
         CellArgs ca{cells_.count, cells_.members, cells_.nc[0], cells_.nc[1], cells_.nc[2], cells_.cap,
                     cells_.inv_cell[0], cells_.inv_cell[1], cells_.inv_cell[2]};
         hipLaunchKernelGGL(commit_kernel, dim3(1), dim3(64), 0, stream_, d_pos_, args, ca, cells_.cell_of,
-                           cells_.overflow, make_box(model_), cells_.enabled ? 1 : 0);
+                           cells_.overflow, make_box(model_), cells_.enabled ? 1 : 0, d_gcm_, pending_cm_group_, pending_cm_[0],
+                           pending_cm_[1], pending_cm_[2]);
         check_hip(hipGetLastError(), "commit_kernel");
         for (const auto& M : pending_moved_) {
             h_xyz_[3 * M.idx] = M.newp.x;
@@ -1425,11 +1461,8 @@ void Engine::sync(bool accept) {
         }
         std::swap(d_q_acc_, d_q_trial_);
         for (int d = 0; d < 3; ++d) dipole_[d] = dipole_trial_[d];
-        if (pending_cm_group_ >= 0) {
+        if (pending_cm_group_ >= 0)
             for (int d = 0; d < 3; ++d) g_cm_[static_cast<size_t>(3 * pending_cm_group_ + d)] = pending_cm_[d];
-            check_hip(hipMemcpy(d_gcm_ + 3 * pending_cm_group_, pending_cm_, sizeof(double) * 3, hipMemcpyHostToDevice),
-                      "copy mass centre");
-        }
     }
     pending_ = false;
     pending_cm_group_ = -1;

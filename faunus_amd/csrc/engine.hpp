@@ -55,6 +55,7 @@ struct alignas(16) DevCoulomb {
     // bucket[b]: index of the first knot >= b / kSplineBuckets (start of the interval search)
     unsigned short bucket[kSplineBuckets + 1];
     int nspl;
+    // last: only the nspl tables in use need be copied
     DevSplineTable spl[kSplMaxTables];
 };
 
@@ -274,7 +275,8 @@ class Engine {
     void build_kvectors();
     void full_q(double2* out);
     void build_cell_list();
-    void launch_delta(const MoveArgs& args, int pair_blocks, int ewald_blocks, bool bond_block);
+    void launch_delta(const MoveArgs& args, int ewald_blocks, bool bond_block);
+    void wait_result();
     void build_group_tables();
     // PBC-safe mass centre of group g around its first atom (Geometry::massCenter)
     void group_mass_center_host(int g, double* cm) const;

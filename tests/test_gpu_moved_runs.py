@@ -1,0 +1,43 @@
+"""Per-move energy changes at the edges of the launch's splits: one to many moved atoms (runs of
+moved atoms, chunks of the phase tables, also with a k list so wide that a chunk holds few
+atoms), particle counts around a block, and cells with fewer and more members than lanes,
+against the oracle."""
+import numpy as np
+import pytest
+
+import faunus_amd as F
+from tests import systems
+from tests.gpu_helpers import build_pair, close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n_beads,n_total,moved,kmax", [
+    (20, 255, 1, 5), (20, 256, 2, 5), (20, 257, 4, 7), (20, 258, 5, 7), (30, 300, 8, 9), (30, 300, 9, 9),
+    (40, 513, 17, 6), (40, 90, 39, 5), (24, 120, 9, 22)])
+def test_several_moved_atoms(n_beads, n_total, moved, kmax):
+    cfg, xyz, q, ids, g, _ = systems.polyelectrolyte(n_beads, n_total, seed=7, kmax=kmax)
+    orc, eng, e_cpu, e_gpu = build_pair((cfg, xyz, q, ids, g), F.Engine)
+    rng = np.random.default_rng(moved)
+    rel = np.sort(rng.choice(n_beads, moved, replace=False)).astype(int)
+    box = cfg["geometry"]["length"]
+    new = xyz[rel] + 0.5 * (2 * rng.random((moved, 3)) - 1)
+    new -= box * np.round(new / box)
+    change = dict(groups=[dict(group_index=0, internal=True, relative_atom_indices=list(rel))])
+    eng.stage_trial(rel, new)
+    got = eng.delta_u(change)
+    want = orc.energy_change(change, rel, new)
+    for a, b in zip(got, want):
+        assert close(a, b, floor=abs(e_cpu)).all(), (a, b)
+    eng.sync(True)
+    assert close(eng.check_q()[0], 0.0).all()  # the accepted Q(k) against a full update
+
+
+@pytest.mark.parametrize("n_pairs,box", [(60, 48.0), (400, 48.0), (800, 48.0)])
+def test_cell_occupancies(n_pairs, box):
+    """4 x 4 x 4 cells of 12 A holding 2, 13 and 25 ions on average (4, 16 and 32 lanes)."""
+    orc, eng, e_cpu, e_gpu = build_pair(systems.nacl_lj(n_pairs=n_pairs, box=box, kmax=4, seed=2), F.Engine)
+    rec = orc.run_translate(60, seed=3)
+    out = eng.replay_translate(rec["group"], rec["index"], rec["xyz"], rec["u"])
+    assert close(out["du"], rec["du"], floor=max(1.0, abs(e_cpu))).all()
+    assert np.array_equal(out["accepted"], rec["accepted"])
