@@ -33,10 +33,14 @@ def test_several_moved_atoms(n_beads, n_total, moved, kmax):
     assert close(eng.check_q()[0], 0.0).all()  # the accepted Q(k) against a full update
 
 
-@pytest.mark.parametrize("n_pairs,box", [(60, 48.0), (400, 48.0), (800, 48.0)])
-def test_cell_occupancies(n_pairs, box):
+@pytest.mark.parametrize("n", [128, 832, 1600])
+def test_cell_occupancies(n):
     """4 x 4 x 4 cells of 12 A holding 2, 13 and 25 ions on average (4, 16 and 32 lanes)."""
-    orc, eng, e_cpu, e_gpu = build_pair(systems.nacl_lj(n_pairs=n_pairs, box=box, kmax=4, seed=2), F.Engine)
+    cfg = systems.nacl_lj(n_pairs=20, box=48.0, kmax=4, seed=2)[0]
+    xyz = systems.lattice_positions(n, 48.0, 3.0, np.random.default_rng(n))
+    ids = np.arange(n, dtype=np.int32) % 2
+    groups = dict(begin=[0], size=[n], molid=[0])
+    orc, eng, e_cpu, e_gpu = build_pair((cfg, xyz, np.where(ids == 0, 1.0, -1.0), ids, groups), F.Engine)
     rec = orc.run_translate(60, seed=3)
     out = eng.replay_translate(rec["group"], rec["index"], rec["xyz"], rec["u"])
     assert close(out["du"], rec["du"], floor=max(1.0, abs(e_cpu))).all()
