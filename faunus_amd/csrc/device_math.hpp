@@ -70,12 +70,14 @@ __device__ __forceinline__ double spline_window(const double* __restrict__ knots
     }
     double k = below <= 1 ? v[0] : (below == 2 ? v[1] : (below == 3 ? v[2] : v[3]));
     int pos = lo + below - 1;
-    if (steps > 4 || (below == 0 && lo > 0) || pos > n - 2) {
+    if (steps > 4) { // uniform over the wave for one table
         for (int s = 4; s < steps; ++s) pos += (lo + s < n && knots[lo + s] < x) ? 1 : 0;
-        pos = pos < 0 ? 0 : (pos > n - 2 ? n - 2 : pos);
+        pos = pos < 0 ? 0 : pos;
         k = knots[pos];
     }
-    pos = pos < 0 ? 0 : pos;
+    // lo's knot lies below x unless it is the first one; past the last interval (x beyond the
+    // last knot) the value is not used, only its address kept in range
+    pos = pos < 0 ? 0 : (pos > n - 2 ? n - 2 : pos);
     const double2* c = reinterpret_cast<const double2*>(coeff + 6 * pos);
     const double2 c01 = c[0], c23 = c[1], c45 = c[2];
     const double z = x - k;

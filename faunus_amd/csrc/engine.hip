@@ -723,7 +723,9 @@ void Engine::upload_potentials() {
                 const double span = s.table.knots.back() - T.x0;
                 T.inv_w = kSplBuckets / span;
                 for (int k = 0; k <= kSplBuckets; ++k) {
-                    const double x = T.x0 + k / T.inv_w;
+                    // a little below the bucket's edge, so that the knot before the first one
+                    // found lies below every r2 that rounds into the bucket
+                    const double x = T.x0 + k / T.inv_w - 1e-9 * span;
                     T.bucket[k] = static_cast<unsigned char>(
                         std::lower_bound(s.table.knots.begin(), s.table.knots.end(), x) - s.table.knots.begin());
                 }

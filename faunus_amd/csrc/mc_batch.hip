@@ -94,6 +94,7 @@ __global__ __launch_bounds__(kThreads) void mc_advance_kernel(ReplicaState* __re
             for (int i = tid; i < kSTable; i += kThreads) s_stab[i] = S.stab[i];
     }
     const CoulF cf = coul_f32(s_coul);
+    const int form = pair_form(s_coul, S.terms, kF32);
 
     // this thread's chunk of k-vectors and their running structure factors
     const int k0 = tid * kpt;
@@ -161,14 +162,16 @@ __global__ __launch_bounds__(kThreads) void mc_advance_kernel(ReplicaState* __re
             fb = fixed_pos(po.x, po.y, po.z, po.w, inv);
         }
         if (!kCells) {
-            if (kF32) {
-                pair_row_f32<kThreads>(pos32, meta, 0, n, i, -1, true, s_pairs_f + ti * nt, cf, s_stab, S.terms, hf,
-                                       fa, fb, &s_nhot, s_hot, 0, e_new, e_old);
-            } else {
-                const Box b{{L, L, L}, {half, half, half}};
-                pair_row_f64<kThreads>(pos, meta, 0, n, i, -1, true, s_pairs + ti * nt, s_coul, S.terms, b, nx_, ny_, nz_,
-                                       po.x, po.y, po.z, po.w, e_new, e_old);
-            }
+            with_form(form, [&](auto f) __attribute__((always_inline)) {
+                if (kF32) {
+                    pair_row_f32<kThreads, f()>(pos32, meta, 0, n, i, -1, true, s_pairs_f + ti * nt, cf, s_stab, S.terms, hf,
+                                                fa, fb, &s_nhot, s_hot, 0, e_new, e_old);
+                } else {
+                    const Box b{{L, L, L}, {half, half, half}};
+                    pair_row_f64<kThreads, f()>(pos, meta, 0, n, i, -1, true, s_pairs + ti * nt, s_coul, S.terms, b, nx_,
+                                                ny_, nz_, po.x, po.y, po.z, po.w, e_new, e_old);
+                }
+            });
         } else {
             // 27-cell stencils around the new (st=0) and old (st=1) position
             const int lanes_per = kThreads / 54 > 0 ? kThreads / 54 : 1;

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 #include <vector>
 
 #include "device_math.hpp"
@@ -123,7 +124,8 @@ __host__ __device__ inline uint32_t fixed_coord(double x, double s) {
 #ifdef __HIP_DEVICE_COMPILE__
     // adding 1.5 x 2^52 rounds to the nearest integer and leaves it, modulo 2^32, in the low
     // word (no 64-bit conversion); the product is rounded first, as on the host
-    const double v = __dadd_rn(__dmul_rn(x, s), 6755399441055744.0);
+#pragma clang fp contract(off)
+    const double v = x * s + 6755399441055744.0;
     return static_cast<uint32_t>(__double_as_longlong(v)) + 0x80000000u;
 #else
     return static_cast<uint32_t>(static_cast<long long>(rint(x * s)) + 2147483648ll);
@@ -168,7 +170,8 @@ __device__ __forceinline__ float dist2_fix(const FixPos& a, const FixPos& b, flo
     const float dx = static_cast<float>(static_cast<int>(a.x - b.x)) * h;
     const float dy = static_cast<float>(static_cast<int>(a.y - b.y)) * h;
     const float dz = static_cast<float>(static_cast<int>(a.z - b.z)) * h;
-    return dx * dx + dy * dy + dz * dz;
+    // one order of the fused sums in every kernel, whatever the code around it
+    return __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
 }
 
 // Hot pairs (inside their type pair's hot radius, hot_radius2) are evaluated again in
@@ -254,12 +257,91 @@ __device__ __forceinline__ float pair_energy_ft(const DevPairF& p, const CoulF& 
     return u;
 }
 
+// The pair forms with straight-line code of their own: hard spheres or Lennard-Jones plus
+// an Ewald or Fanourgakis term with its short-range table.  In the other forms every switch
+// (tables, terms, scheme) is a branch in each pair energy, so that the LDS latencies of the
+// neighbours a lane holds follow one another; without branches they overlap.
+enum PairForm : int { kFormAny = 0, kFormHS = 1, kFormLJ = 2 };
+
+__device__ __forceinline__ int pair_form(const DevCoulomb& c, int terms, bool f32) {
+    const bool table = c.nspl == 0 && (c.scheme == kCoulEwald || c.scheme == kCoulFanourgakis) && (f32 || c.splined);
+    return !table ? kFormAny : (terms == kTermHS ? kFormHS : (terms == kTermLJ ? kFormLJ : kFormAny));
+}
+
+__device__ __forceinline__ void materialize(float& x) { asm("" : "+v"(x)); }
+__device__ __forceinline__ void materialize(double& x) { asm("" : "+v"(x)); }
+
+// pair_energy_ft of a form: the same arithmetic, its fused operations spelled out.
+template <int kForm>
+__device__ __forceinline__ float pair_f32(const DevPairF& p, const CoulF& c, const float4* __restrict__ tab, int terms,
+                                          float qa, float qb, float r2, bool& hot) {
+    if constexpr (kForm == kFormAny) {
+        return pair_energy_ft(p, c, tab, terms, qa, qb, r2, hot);
+    } else {
+#pragma clang fp contract(off)
+        const float4 pa = reinterpret_cast<const float4*>(&p)[0]; // lj_s2, lj_e4, wca_s2, wca_e4
+        const float4 pb = reinterpret_cast<const float4*>(&p)[1]; // hs_s2, coul, spl (bits), hot_r2
+        hot = r2 < pb.w;
+        float u;
+        if constexpr (kForm == kFormLJ) {
+            float x = pa.x * __builtin_amdgcn_rcpf(r2);
+            x = x * x * x;
+            u = pa.y * __builtin_fmaf(x, x, -x);
+        } else {
+            u = (r2 < pb.x * kHsSure) ? __builtin_huge_valf() : 0.0f;
+        }
+        const float ir = __builtin_amdgcn_rsqf(r2);
+        const float r = r2 * ir;
+        const float t = r * c.rc_inv * static_cast<float>(kSTable);
+        int i = static_cast<int>(t);
+        i = i > kSTable - 1 ? kSTable - 1 : i;
+        i = i < 0 ? 0 : i;
+        const float f = t - static_cast<float>(i);
+        const float4 k = tab[i];
+        const float sv = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(k.w, f, k.z), f, k.y), f, k.x);
+        float e = c.lB * (qa * qb * ir * sv);
+        materialize(e); // selected, not branched around
+        return u + (r < c.rc && pb.y != 0.0f ? e : 0.0f);
+    }
+}
+
+// pair_energy_t of a form: the same arithmetic.
+template <int kForm>
+__device__ __forceinline__ double pair_f64(const DevPair& p, const DevCoulomb& c, double qa, double qb, double r2,
+                                           int terms) {
+    if constexpr (kForm == kFormAny) {
+        return pair_energy_t(p, c, qa, qb, r2, terms);
+    } else {
+        double u;
+        if constexpr (kForm == kFormLJ) {
+            double x = p.lj_s2 / r2;
+            x = x * x * x;
+            u = p.lj_e4 * (x * x - x);
+            materialize(u);
+            u = p.lj_e4 != 0.0 ? u : 0.0;
+        } else {
+            u = (r2 < p.hs_s2) ? __builtin_huge_val() : 0.0;
+        }
+        const double r = sqrt(r2) + 2.220446049250313e-16;
+        double e = c.lB * (qa * qb / r * coulomb_spline(c, r * c.rc_inv));
+        materialize(e);
+        return u + (r < c.rc && p.coul != 0.0 ? e : 0.0);
+    }
+}
+
+// Calls f(form) with the pair form as a compile-time constant.
+template <class Fn> __device__ __forceinline__ void with_form(int form, Fn&& f) {
+    if (form == kFormHS) f(std::integral_constant<int, kFormHS>{});
+    else if (form == kFormLJ) f(std::integral_constant<int, kFormLJ>{});
+    else f(std::integral_constant<int, kFormAny>{});
+}
+
 // Pair sums of one moved particle, at its new (a) and old (b) position, against every
 // particle j in [jb, n) except `skip`; pairs inside group g count only if same_ok.
-// Lanes stride over j; each lane loads kU neighbours before evaluating them.  FP32
-// terms are summed in FP32 per block of kU and then in FP64; hot pairs go to the queue
-// (hot_n, hot_q) with tag = moved atom << 1.
-template <int kThreads>
+// Lanes stride over j; each lane loads kU neighbours before evaluating them, whole waves
+// past the end excepted.  FP32 terms are summed in FP32 per block of kU and then in FP64; hot
+// pairs go to the queue (hot_n, hot_q) with tag = moved atom << 1.
+template <int kThreads, int kForm>
 __device__ __forceinline__ void pair_row_f32(const FixPos* __restrict__ pos32, const uint32_t* __restrict__ meta, int jb,
                                              int n, int skip, int g, bool same_ok, const DevPairF* row, const CoulF& c,
                                              const float4* tab, int terms, float h, const FixPos& a, const FixPos& b,
@@ -270,23 +352,32 @@ __device__ __forceinline__ void pair_row_f32(const FixPos* __restrict__ pos32, c
         uint32_t mj[kU];
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const int j = j0 + u * kThreads;
-            pj[u] = j < n ? pos32[j] : FixPos{0u, 0u, 0u, 0.0f};
-            mj[u] = j < n ? meta[j] : 0u;
+            const int j = min(j0 + u * kThreads, n - 1);
+            pj[u] = pos32[j];
+            mj[u] = meta[j];
         }
         float sn = 0.0f, so = 0.0f;
         bool anyhot = false;
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
+        auto add = [&](int u) __attribute__((always_inline)) {
             const int j = j0 + u * kThreads;
             const bool ok = j < n && j != skip && (static_cast<int>(mj[u] >> 8) != g || same_ok);
-            const DevPairF& p = row[ok ? static_cast<int>(mj[u] & 0xffu) : 0];
+            const DevPairF& p = row[static_cast<int>(mj[u] & 0xffu)];
             bool hn, ho;
-            const float un = pair_energy_ft(p, c, tab, terms, a.q, pj[u].q, dist2_fix(a, pj[u], h), hn);
-            const float uo = pair_energy_ft(p, c, tab, terms, a.q, pj[u].q, dist2_fix(b, pj[u], h), ho);
+            const float un = pair_f32<kForm>(p, c, tab, terms, a.q, pj[u].q, dist2_fix(a, pj[u], h), hn);
+            const float uo = pair_f32<kForm>(p, c, tab, terms, a.q, pj[u].q, dist2_fix(b, pj[u], h), ho);
             sn += ok ? un : 0.0f;
             so += ok ? uo : 0.0f;
             anyhot = anyhot || (ok && (hn || ho));
+        };
+        // slots that lie past the end for the wave's first lane are past it for the wave
+        const int slots = __builtin_amdgcn_readfirstlane((n - 1 - j0) / kThreads + 1);
+        if (slots >= kU) {
+#pragma unroll
+            for (int u = 0; u < kU; ++u) add(u);
+        } else {
+            add(0);
+            if (slots > 1) add(1);
+            if (slots > 2) add(2);
         }
         if (anyhot) {
             // a hot pair in this block: every pair of the block goes to the queue for
@@ -318,31 +409,37 @@ __device__ __forceinline__ void pair_row_f32(const FixPos* __restrict__ pos32, c
     }
 }
 
-template <int kThreads>
+template <int kThreads, int kForm>
 __device__ __forceinline__ void pair_row_f64(const double4* __restrict__ pos, const uint32_t* __restrict__ meta, int jb,
                                              int n, int skip, int g, bool same_ok, const DevPair* row,
                                              const DevCoulomb& c, int terms, const Box& box, double ax, double ay,
                                              double az, double bx, double by, double bz, double qa, double& e_new,
                                              double& e_old) {
-    constexpr int kU = 4;
+    constexpr int kU = 2;
     for (int j0 = jb + static_cast<int>(threadIdx.x); j0 < n; j0 += kThreads * kU) {
         double4 pj[kU];
         uint32_t mj[kU];
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const int j = j0 + u * kThreads;
-            pj[u] = j < n ? pos[j] : make_double4(0.0, 0.0, 0.0, 0.0);
-            mj[u] = j < n ? meta[j] : 0u;
+            const int j = min(j0 + u * kThreads, n - 1);
+            pj[u] = pos[j];
+            mj[u] = meta[j];
         }
-#pragma unroll
-        for (int u = 0; u < kU; ++u) {
+        auto add = [&](int u) __attribute__((always_inline)) {
             const int j = j0 + u * kThreads;
             const bool ok = j < n && j != skip && (static_cast<int>(mj[u] >> 8) != g || same_ok);
-            const DevPair& p = row[ok ? static_cast<int>(mj[u] & 0xffu) : 0];
-            const double un = pair_energy_t(p, c, qa, pj[u].w, dist2(box, ax, ay, az, pj[u].x, pj[u].y, pj[u].z), terms);
-            const double uo = pair_energy_t(p, c, qa, pj[u].w, dist2(box, bx, by, bz, pj[u].x, pj[u].y, pj[u].z), terms);
+            const DevPair& p = row[static_cast<int>(mj[u] & 0xffu)];
+            const double un = pair_f64<kForm>(p, c, qa, pj[u].w, dist2(box, ax, ay, az, pj[u].x, pj[u].y, pj[u].z), terms);
+            const double uo = pair_f64<kForm>(p, c, qa, pj[u].w, dist2(box, bx, by, bz, pj[u].x, pj[u].y, pj[u].z), terms);
             e_new += ok ? un : 0.0;
             e_old += ok ? uo : 0.0;
+        };
+        const int slots = __builtin_amdgcn_readfirstlane((n - 1 - j0) / kThreads + 1);
+        if (slots >= kU) {
+#pragma unroll
+            for (int u = 0; u < kU; ++u) add(u);
+        } else {
+            add(0);
         }
     }
 }

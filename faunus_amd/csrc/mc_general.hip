@@ -79,7 +79,7 @@ struct MovedSet {
 // the FP32 form, hot pairs go to the queue (hot_n, hot_q).
 // kExcl: the system has pair exclusions (looked up per pair inside the moved group);
 // without them the loop over the neighbours is straight-line code.
-template <int kThreads, int kB, bool kF32, bool kExcl, bool kCut>
+template <int kThreads, int kB, bool kF32, bool kExcl, bool kCut, int kForm>
 __device__ __forceinline__ void moved_block(int base, int je, const MovedSet& ms, const uint32_t* __restrict__ meta,
                                             const FixPos* __restrict__ pos32, const double4* __restrict__ pos,
                                             const DevPairF* s_pairs_f, const DevPair* s_pairs, int nt, const CoulF& cf,
@@ -139,8 +139,8 @@ __device__ __forceinline__ void moved_block(int base, int je, const MovedSet& ms
                 const bool ok = pair_ok(u, okn, oko);
                 const DevPairF& p = row[ok ? static_cast<int>(mj[u] & 0xffu) : 0];
                 bool hn, ho;
-                const float un = pair_energy_ft(p, cf, s_stab, terms, fa.q, pf[u].q, dist2_fix(fa, pf[u], hf), hn);
-                const float uo = pair_energy_ft(p, cf, s_stab, terms, fa.q, pf[u].q, dist2_fix(fb, pf[u], hf), ho);
+                const float un = pair_f32<kForm>(p, cf, s_stab, terms, fa.q, pf[u].q, dist2_fix(fa, pf[u], hf), hn);
+                const float uo = pair_f32<kForm>(p, cf, s_stab, terms, fa.q, pf[u].q, dist2_fix(fb, pf[u], hf), ho);
                 sn += okn ? un : 0.0f;
                 so += oko ? uo : 0.0f;
                 anyhot = anyhot || (okn && hn) || (oko && ho);
@@ -185,9 +185,9 @@ __device__ __forceinline__ void moved_block(int base, int je, const MovedSet& ms
                                       : uu != 0;
                 const DevPair& p = row[ok ? static_cast<int>(mj[u] & 0xffu) : 0];
                 const double un =
-                    pair_energy_t(p, s_coul, A.w, pj[u].w, dist2(box, A.x, A.y, A.z, pj[u].x, pj[u].y, pj[u].z), terms);
+                    pair_f64<kForm>(p, s_coul, A.w, pj[u].w, dist2(box, A.x, A.y, A.z, pj[u].x, pj[u].y, pj[u].z), terms);
                 const double uo =
-                    pair_energy_t(p, s_coul, B.w, pj[u].w, dist2(box, B.x, B.y, B.z, pj[u].x, pj[u].y, pj[u].z), terms);
+                    pair_f64<kForm>(p, s_coul, B.w, pj[u].w, dist2(box, B.x, B.y, B.z, pj[u].x, pj[u].y, pj[u].z), terms);
                 sn += (ok && !(use[u] & 4)) ? un : 0.0;
                 so += (ok && !(use[u] & 8)) ? uo : 0.0;
             }
@@ -286,6 +286,7 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
             for (int i = tid; i < kSTable; i += kThreads) s_stab[i] = S.stab[i];
     }
     const CoulF cf = coul_f32(s_coul);
+    const int form = pair_form(s_coul, S.terms, kF32);
 
     const int k0 = kb + tid * kpt;
     double2 q[kMaxKPT];
@@ -549,51 +550,56 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
             // one moved atom: the row sums with the moved coordinates in registers
             const double4 A = s_new[0], B = s_old[0];
             const int ta = s_mt[0];
-            if (kF32) {
-                pair_row_f32<kThreads>(pos32, meta, jb, je, P.mlo, g, same_ok, s_pairs_f + ta * nt, cf, s_stab, terms, hf,
-                                       fixed_pos(A.x, A.y, A.z, A.w, inv), fixed_pos(B.x, B.y, B.z, B.w, inv), &s_nhot,
-                                       s_hot, 0, e_new, e_old);
-            } else {
-                pair_row_f64<kThreads>(pos, meta, jb, je, P.mlo, g, same_ok, s_pairs + ta * nt, s_coul, terms, box, A.x,
-                                       A.y, A.z, B.x, B.y, B.z, A.w, e_new, e_old);
-            }
+            with_form(form, [&](auto f) __attribute__((always_inline)) {
+                if (kF32) {
+                    pair_row_f32<kThreads, f()>(pos32, meta, jb, je, P.mlo, g, same_ok, s_pairs_f + ta * nt, cf, s_stab, terms,
+                                                hf, fixed_pos(A.x, A.y, A.z, A.w, inv), fixed_pos(B.x, B.y, B.z, B.w, inv),
+                                                &s_nhot, s_hot, 0, e_new, e_old);
+                } else {
+                    pair_row_f64<kThreads, f()>(pos, meta, jb, je, P.mlo, g, same_ok, s_pairs + ta * nt, s_coul, terms, box,
+                                                A.x, A.y, A.z, B.x, B.y, B.z, A.w, e_new, e_old);
+                }
+            });
         } else if (m > 0) {
             if (!kCells) {
                 // blocks of kB neighbours per lane (kB from 8 down to 1 as the slice
                 // runs out, so that few lanes sit idle on short slices)
                 const MovedSet ms{P.mlo,    P.mhi, m,    g,    same_ok, s_new, s_old,   fixlds ? s_fnew : nullptr,
                                   s_fold,   inv,   s_mt, excl_off, excl, gcut,  s_cm[0], s_cm[1]};
-                auto blocks = [&](auto excl_tag, auto cut_tag) {
+                auto blocks = [&](auto excl_tag, auto cut_tag, auto form_tag) {
                     constexpr bool kX = decltype(excl_tag)::value;
                     constexpr bool kC = decltype(cut_tag)::value;
+                    constexpr int kP = decltype(form_tag)::value;
                     int base = jb;
                     while (base < je) {
                         const int rem = je - base;
                         if (kF32 && rem >= 8 * kThreads) {
-                            moved_block<kThreads, 8, kF32, kX, kC>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
+                            moved_block<kThreads, 8, kF32, kX, kC, kP>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
                                                                s_stab, s_coul, terms, box, hf, &s_nhot, s_hot, e_new, e_old);
                             base += 8 * kThreads;
                         } else if (rem >= 4 * kThreads) {
-                            moved_block<kThreads, 4, kF32, kX, kC>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
+                            moved_block<kThreads, 4, kF32, kX, kC, kP>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
                                                                s_stab, s_coul, terms, box, hf, &s_nhot, s_hot, e_new, e_old);
                             base += 4 * kThreads;
                         } else if (rem > kThreads) {
-                            moved_block<kThreads, 2, kF32, kX, kC>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
+                            moved_block<kThreads, 2, kF32, kX, kC, kP>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
                                                                s_stab, s_coul, terms, box, hf, &s_nhot, s_hot, e_new, e_old);
                             base += 2 * kThreads;
                         } else {
-                            moved_block<kThreads, 1, kF32, kX, kC>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
+                            moved_block<kThreads, 1, kF32, kX, kC, kP>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
                                                                s_stab, s_coul, terms, box, hf, &s_nhot, s_hot, e_new, e_old);
                             base += kThreads;
                         }
                     }
                 };
+                using Any = std::integral_constant<int, kFormAny>;
                 if (excl_off != nullptr) {
-                    if (cutg) blocks(std::true_type{}, std::true_type{});
-                    else blocks(std::true_type{}, std::false_type{});
+                    if (cutg) blocks(std::true_type{}, std::true_type{}, Any{});
+                    else blocks(std::true_type{}, std::false_type{}, Any{});
+                } else if (cutg) {
+                    blocks(std::false_type{}, std::true_type{}, Any{});
                 } else {
-                    if (cutg) blocks(std::false_type{}, std::true_type{});
-                    else blocks(std::false_type{}, std::false_type{});
+                    with_form(form, [&](auto f) __attribute__((always_inline)) { blocks(std::false_type{}, std::false_type{}, f); });
                 }
             } else {
               // stencils of (2r+1)^3 cells (cells of at least range / r) around each moved
