@@ -12,49 +12,23 @@
 #include "device_math.hpp"
 #include "mc_batch.hpp"
 #include "mc_common.hpp"
+#include "mc_ladder.hpp"
 #include "philox.hpp"
 
 namespace fmc {
 namespace {
 
-// One round of neighbour exchanges in one ladder (ParallelTempering, move.cpp:844-965):
-// rungs k, k+1 for k of the round's parity, accepted with min(1, exp((b_a - b_b)(E_a -
-// E_b))) on a Philox deviate of (round, ladder, k); an accepted swap exchanges the betas
-// and the rung slots.
-__device__ void swap_ladder_rungs(ReplicaState* states, int b, int m, int* rung_slot, int l, unsigned long long seed,
-                                  unsigned long long round, unsigned long long* counters) {
-    for (int k = static_cast<int>(round & 1); k + 1 < m; k += 2) {
-        const int sa = rung_slot[b + k], sb = rung_slot[b + k + 1];
-        ReplicaState& A = states[sa];
-        ReplicaState& B = states[sb];
-        const double x = (A.beta - B.beta) * (A.energy - B.energy);
-        const Philox4 r = philox4x32_10(static_cast<uint32_t>(round), static_cast<uint32_t>(round >> 32),
-                                        static_cast<uint32_t>(l), 0x5a5a0000u + static_cast<uint32_t>(k),
-                                        static_cast<uint32_t>(seed), static_cast<uint32_t>(seed >> 32));
-        const double u = (static_cast<double>(r.v[0] >> 5) * 67108864.0 + static_cast<double>(r.v[1] >> 6)) *
-                         1.1102230246251565e-16;
-        atomicAdd(&counters[0], 1ull);
-        if (x >= 0.0 || u < exp(x)) {
-            const double tb = A.beta;
-            A.beta = B.beta;
-            B.beta = tb;
-            rung_slot[b + k] = sb;
-            rung_slot[b + k + 1] = sa;
-            atomicAdd(&counters[1], 1ull);
-        }
-    }
-}
-
 template <int kThreads, int kMaxKPT, bool kCells, bool kF32>
 __global__ __launch_bounds__(kThreads) void mc_advance_kernel(ReplicaState* __restrict__ states,
                                                                const long long* __restrict__ moves,
                                                                TraceEntry* __restrict__ trace, int trace_cap,
-                                                               const LadderRun* __restrict__ ladders) {
-    ReplicaState& S = states[blockIdx.x];
-    const long long M = moves[blockIdx.x];
+                                                               const LadderRun* __restrict__ ladders, ReplicaMap map) {
+    const int rep = map.first + map.id[blockIdx.x];
+    ReplicaState& S = states[rep];
+    const long long M = moves[rep];
     // free-running ladders: every replica takes part in its ladder's barriers, also one
     // with no moves or an error
-    const int n_iv = ladders != nullptr ? ladders->intervals[blockIdx.x] : 1;
+    const int n_iv = ladders != nullptr ? ladders->intervals[rep] : 1;
     if (ladders == nullptr && (M <= 0 || S.error)) return;
     __shared__ DevPair s_pairs[kMaxTypes * kMaxTypes];
     __shared__ DevPairF s_pairs_f[kF32 ? kMaxTypes * kMaxTypes : 1];
@@ -291,7 +265,7 @@ __global__ __launch_bounds__(kThreads) void mc_advance_kernel(ReplicaState* __re
             s_accept = acc ? 1 : 0;
             if (kF32) s_nhot = 0; // every thread has read the queue before the reduction
             if (trace && t < trace_cap) {
-                TraceEntry& T = trace[static_cast<size_t>(blockIdx.x) * trace_cap + t];
+                TraceEntry& T = trace[static_cast<size_t>(rep) * trace_cap + t];
                 T.index = i;
                 T.accepted = acc ? 1 : 0;
                 T.du = du;
@@ -385,34 +359,7 @@ __global__ __launch_bounds__(kThreads) void mc_advance_kernel(ReplicaState* __re
         S.e_samples = e_samples;
         S.e_sum = e_sum;
         S.e_sum2 = e_sum2;
-        const int l = ladders != nullptr ? ladders->ladder_of[blockIdx.x] : -1;
-        if (l >= 0) {
-            const LadderRun& lr = *ladders;
-            // the ladder's barrier: the energy above is published before the arrival; the
-            // last replica to arrive swaps the rungs, the others wait for its release
-            __threadfence();
-            const unsigned target = static_cast<unsigned>(lr.size[l]) * static_cast<unsigned>(iv + 1);
-            if (atomicAdd(&lr.arrive[l], 1u) + 1u == target) {
-                __threadfence();
-                swap_ladder_rungs(states, lr.begin[l], lr.size[l], lr.rung_slot, l, lr.seed,
-                                  lr.round0 + static_cast<unsigned long long>(iv), lr.counters);
-                __threadfence();
-                __hip_atomic_store(&lr.gen[l], static_cast<unsigned>(iv + 1), __ATOMIC_RELEASE,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                long long spins = 0;
-                while (__hip_atomic_load(&lr.gen[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
-                       static_cast<unsigned>(iv + 1)) {
-                    if (++spins > lr.spin_limit) {
-                        atomicMax(&S.error, 2); // a rung did not arrive: this replica stops
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(20);
-                }
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            }
-            beta = __hip_atomic_load(&S.beta, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        if (ladders != nullptr) ladder_barrier(*ladders, rep, states, S, iv, beta);
     }
     move0 += static_cast<unsigned long long>(t_done);
     __syncthreads(); // the interval's state and error are written before the next interval reads them
@@ -444,7 +391,7 @@ __global__ void ladder_swap_kernel(ReplicaState* states, const int* ladder_begin
 
 template <int kThreads, int kMaxKPT, bool kCells, bool kF32>
 void launch_advance(int grid, size_t lds, hipStream_t st, ReplicaState* s, const long long* m, TraceEntry* tr, int cap,
-                    const LadderRun* lr) {
+                    const LadderRun* lr, ReplicaMap map) {
     auto fn = mc_advance_kernel<kThreads, kMaxKPT, kCells, kF32>;
     // dynamic LDS: what the static LDS leaves of the CU's 160 KB, at most 96 KB (set once)
     static size_t limit = 0;
@@ -458,7 +405,7 @@ void launch_advance(int grid, size_t lds, hipStream_t st, ReplicaState* s, const
     }
     if (lds > limit) throw std::runtime_error("k-vector table too large for LDS");
     if (lr == nullptr) {
-        hipLaunchKernelGGL(fn, dim3(grid), dim3(kThreads), lds, st, s, m, tr, cap, lr);
+        hipLaunchKernelGGL(fn, dim3(grid), dim3(kThreads), lds, st, s, m, tr, cap, lr, map);
         return;
     }
     // ladders wait for each other: every workgroup must be resident at once
@@ -470,7 +417,7 @@ void launch_advance(int grid, size_t lds, hipStream_t st, ReplicaState* s, const
               "occupancy");
     if (per_cu * prop.multiProcessorCount < grid)
         throw std::runtime_error("run_ladders: the replicas cannot all be resident at once");
-    void* args[] = {&s, &m, &tr, &cap, &lr};
+    void* args[] = {&s, &m, &tr, &cap, &lr, &map};
     check_hip(hipLaunchCooperativeKernel(reinterpret_cast<const void*>(fn), dim3(grid), dim3(kThreads), args,
                                          static_cast<unsigned>(lds), st),
               "mc_advance_kernel cooperative launch");
@@ -478,13 +425,13 @@ void launch_advance(int grid, size_t lds, hipStream_t st, ReplicaState* s, const
 
 template <int kThreads, int kMaxKPT>
 void dispatch_cells(bool cells, bool f32, int grid, size_t lds, hipStream_t st, ReplicaState* s, const long long* m,
-                    TraceEntry* tr, int cap, const LadderRun* lr) {
+                    TraceEntry* tr, int cap, const LadderRun* lr, const ReplicaMap& map) {
     if (cells) {
-        if (f32) launch_advance<kThreads, kMaxKPT, true, true>(grid, lds, st, s, m, tr, cap, lr);
-        else launch_advance<kThreads, kMaxKPT, true, false>(grid, lds, st, s, m, tr, cap, lr);
+        if (f32) launch_advance<kThreads, kMaxKPT, true, true>(grid, lds, st, s, m, tr, cap, lr, map);
+        else launch_advance<kThreads, kMaxKPT, true, false>(grid, lds, st, s, m, tr, cap, lr, map);
     } else {
-        if (f32) launch_advance<kThreads, kMaxKPT, false, true>(grid, lds, st, s, m, tr, cap, lr);
-        else launch_advance<kThreads, kMaxKPT, false, false>(grid, lds, st, s, m, tr, cap, lr);
+        if (f32) launch_advance<kThreads, kMaxKPT, false, true>(grid, lds, st, s, m, tr, cap, lr, map);
+        else launch_advance<kThreads, kMaxKPT, false, false>(grid, lds, st, s, m, tr, cap, lr, map);
     }
 }
 
@@ -852,47 +799,75 @@ ReplicaState make_replica_state(Engine& e, bool fp32, unsigned long long seed, i
     return s;
 }
 
+// Replicas with few k-vectors per thread run mc_translate_kernel, the others (K > 8 threads)
+// mc_advance_kernel: a function of the replica alone.
+bool translate_route(const ReplicaState& s) { return s.nk <= 8 * advance_threads(s); }
+
+// 512 threads where they hold the k-vectors at 8 per thread, except with a cell list of so few
+// members that 256 threads take one each and so few k-vectors that 256 threads hold them at 8:
+// there a smaller workgroup's barriers are cheaper (400 moves of 1000 Na/Cl, 2.9 members per cell:
+// 2.52 against 2.68 ms; of 1600 ions, 4.7: 2.12 against 2.26), while 800 moves of 200 ions (7.4) take
+// 4.12 against 3.59 ms and 400 of 3000 Na/Cl with K = 2900 4.04 against 2.69.
 int advance_threads(const ReplicaState& s) {
     if (s.threads) return s.threads;
-    return (!s.cells && s.nk <= 8 * 512) ? 512 : 256;
+    if (s.nk > 8 * 512) return 256;
+    if (!s.cells || s.nk > 8 * 256) return 512;
+    return 54LL * s.n > 256LL * s.nc0 * s.nc1 * s.nc2 ? 512 : 256;
 }
 
 void launch_advance(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
                     TraceEntry* trace, int trace_cap, hipStream_t stream, const LadderRun* ladders) {
-    const LadderRun* lr = ladders;
-    // one launch per run of replicas with the same workgroup size (a function of each
-    // replica alone, so that a replica's arithmetic does not depend on its batch)
-    int first = 0;
-    while (first < count) {
-        const int threads = advance_threads(h_states[first]);
-        int last = first;
-        int maxkpt = 0, maxnk = 0, maxw = 0;
-        while (last < count && advance_threads(h_states[last]) == threads) {
-            const ReplicaState& s = h_states[last];
-            if (s.cells != h_states[first].cells) throw std::runtime_error("replicas of one launch must agree on the cell list");
-            maxkpt = std::max(maxkpt, (s.nk + threads - 1) / threads);
-            maxnk = std::max(maxnk, s.nk);
-            maxw = std::max(maxw, 2 * s.ncut + 1);
-            ++last;
-        }
-        if (maxkpt > 68) throw std::runtime_error("too many k-vectors per replica for the device MC (max 68 per thread)");
-        const size_t lds =
-            sizeof(int) * static_cast<size_t>((maxnk + 3) & ~3) + sizeof(double2) * 6 * static_cast<size_t>(maxw);
-        if (lds > 96 * 1024) throw std::runtime_error("k-vector table too large for LDS");
-        const bool cells = h_states[first].cells != 0;
-        const int grid = last - first;
-        ReplicaState* ds = d_states + first;
-        const long long* dm = d_moves + first;
-        TraceEntry* tr = trace ? trace + static_cast<size_t>(first) * trace_cap : nullptr;
-        if (lr != nullptr && (first != 0 || last != count))
-            throw std::runtime_error("run_ladders: every replica must take the same workgroup size");
-        if (threads == 512) dispatch_cells<512, 8>(cells, f32, grid, lds, stream, ds, dm, tr, trace_cap, lr);
-        else if (maxkpt <= 8) dispatch_cells<256, 8>(cells, f32, grid, lds, stream, ds, dm, tr, trace_cap, lr);
-        else if (maxkpt <= 32) dispatch_cells<256, 32>(cells, f32, grid, lds, stream, ds, dm, tr, trace_cap, lr);
-        else dispatch_cells<256, 68>(cells, f32, grid, lds, stream, ds, dm, tr, trace_cap, lr);
-        check_hip(hipGetLastError(), "mc_advance_kernel launch");
-        first = last;
+    // workgroup size and kernel of each replica, functions of the replica alone (so that its
+    // arithmetic does not depend on its batch), except that the replicas of a ladder launch
+    // with cell lists take 256 threads, and the kernel for any K, when they do not agree
+    std::vector<int> threads(static_cast<size_t>(count));
+    std::vector<char> translate(static_cast<size_t>(count));
+    bool same = true, cells = true, all = true;
+    for (int r = 0; r < count; ++r) {
+        const ReplicaState& s = h_states[r];
+        if (s.cells != h_states[0].cells) throw std::runtime_error("replicas of one launch must agree on the cell list");
+        threads[static_cast<size_t>(r)] = advance_threads(s);
+        same = same && threads[static_cast<size_t>(r)] == threads[0];
+        cells = cells && s.cells != 0;
     }
+    if (ladders != nullptr && !same) {
+        if (!cells) throw std::runtime_error("run_ladders: every replica must take the same workgroup size");
+        std::fill(threads.begin(), threads.end(), 256);
+    }
+    if (ladders != nullptr && count > ReplicaMap::kMax)
+        throw std::runtime_error("run_ladders: the replicas cannot all be resident at once");
+    for (int r = 0; r < count; ++r) {
+        const int kpt = (h_states[r].nk + threads[static_cast<size_t>(r)] - 1) / threads[static_cast<size_t>(r)];
+        if (kpt > 68) throw std::runtime_error("too many k-vectors per replica for the device MC (max 68 per thread)");
+        translate[static_cast<size_t>(r)] = kpt <= 8 ? 1 : 0;
+        all = all && kpt <= 8;
+    }
+    if (ladders != nullptr && !all) std::fill(translate.begin(), translate.end(), 0);
+    auto table_bytes = [&](const std::vector<int>& ids) {
+        int nk = 0, width = 0;
+        for (int r : ids) {
+            nk = std::max(nk, h_states[r].nk);
+            width = std::max(width, 2 * h_states[r].ncut + 1);
+        }
+        return sizeof(int) * static_cast<size_t>((nk + 3) & ~3) + sizeof(double2) * 6 * static_cast<size_t>(width);
+    };
+    for (int r = 0; r < count; ++r)
+        if (table_bytes({r}) > 96 * 1024) throw std::runtime_error("k-vector table too large for LDS");
+    launch_by_route(count, [&](int r) { return 2 * threads[static_cast<size_t>(r)] + translate[static_cast<size_t>(r)]; },
+                    [&](const std::vector<int>& ids, const ReplicaMap& map) {
+        const size_t first = static_cast<size_t>(ids[0]);
+        if (translate[first]) {
+            launch_translate(h_states, ids, map, threads[first], d_states, d_moves, f32, trace, trace_cap, stream, ladders);
+            return;
+        }
+        int kpt = 0;
+        for (int r : ids) kpt = std::max(kpt, (h_states[r].nk + 255) / 256);
+        const int grid = static_cast<int>(ids.size());
+        const size_t lds = table_bytes(ids);
+        if (kpt <= 32) dispatch_cells<256, 32>(cells, f32, grid, lds, stream, d_states, d_moves, trace, trace_cap, ladders, map);
+        else dispatch_cells<256, 68>(cells, f32, grid, lds, stream, d_states, d_moves, trace, trace_cap, ladders, map);
+        check_hip(hipGetLastError(), "mc_advance_kernel launch");
+    });
 }
 
 int Batch::add_replica(const std::string& config_json, int n, const double* xyz, const double* charge, const int* ids,

@@ -6,6 +6,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <memory>
 #include <string>
@@ -106,6 +107,43 @@ struct ReplicaState {
     int threads;              // workgroup size of the translate-only kernel chosen by the tuner (0: the default rule)
 };
 
+// The replicas of one launch: block b advances replica first + id[b].  By value, so that a launch
+// can take any subset of a batch's replicas without device memory of its own.
+struct ReplicaMap {
+    static constexpr int kMax = 1024;
+    int first;
+    unsigned short id[kMax];
+};
+
+// Calls launch(indices, map) for the replicas of each route (route(r), any int) in turn, at most
+// ReplicaMap::kMax at a time: replicas that take different kernels or workgroup sizes share a
+// batch in any order and make one launch per route, not one per change of route.
+template <class Route, class Launch> void launch_by_route(int count, Route&& route, Launch&& launch) {
+    std::vector<int> of(static_cast<size_t>(count));
+    std::vector<int> routes;
+    for (int r = 0; r < count; ++r) {
+        of[static_cast<size_t>(r)] = route(r);
+        if (std::find(routes.begin(), routes.end(), of[static_cast<size_t>(r)]) == routes.end())
+            routes.push_back(of[static_cast<size_t>(r)]);
+    }
+    for (int k : routes) {
+        std::vector<int> ids;
+        ReplicaMap map{};
+        auto flush = [&]() {
+            if (!ids.empty()) launch(ids, map);
+            ids.clear();
+        };
+        for (int r = 0; r < count; ++r) {
+            if (of[static_cast<size_t>(r)] != k) continue;
+            if (static_cast<int>(ids.size()) == ReplicaMap::kMax || (!ids.empty() && r - map.first > 0xffff)) flush();
+            if (ids.empty()) map.first = r;
+            map.id[ids.size()] = static_cast<unsigned short>(r - map.first);
+            ids.push_back(r);
+        }
+        flush();
+    }
+}
+
 // Free-running temperature ladders in one persistent launch (Batch::run_ladders): replica
 // r runs intervals[r] swap intervals of its moves[r] moves; after each, the replicas of
 // a ladder meet at a barrier in HBM and the last to arrive swaps the ladder's rungs, so
@@ -139,11 +177,17 @@ ReplicaState make_replica_state(Engine& e, bool fp32, unsigned long long seed, i
 // Pair energies at the squared distances r2[n] of types ta, tb with charges qa, qb in the
 // two device forms: FP64 (u64) and FP32 (u32, the device-resident kernels' form).
 void pair_probe(Engine& e, int ta, int tb, double qa, double qb, int n, const double* r2, double* u64, double* u32);
-// Workgroup size of the translate-only kernel for a replica: 512 threads (two waves per
-// SIMD) without a cell list and with K <= 4096, else 256.
+// Workgroup size of the translate-only kernels for a replica (256 or 512 threads), from the
+// replica alone.
 int advance_threads(const ReplicaState& s);
+// Whether mc_translate_kernel advances a replica (at most 8 k-vectors per thread), and its launch
+// of the replicas `ids` (of a batch's h_states) with `threads` per workgroup.
+bool translate_route(const ReplicaState& s);
+void launch_translate(const ReplicaState* h_states, const std::vector<int>& ids, const ReplicaMap& map, int threads,
+                      ReplicaState* d_states, const long long* d_moves, bool f32, TraceEntry* trace, int trace_cap,
+                      hipStream_t stream, const LadderRun* ladders);
 // Persistent launches advancing `count` replicas (states already on the device), one
-// per run of replicas with the same workgroup size.  `ladders` (a device pointer, null
+// per kernel and workgroup size among them.  `ladders` (a device pointer, null
 // for one interval without swaps) makes it one cooperative launch of free-running
 // ladders.
 void launch_advance(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
@@ -158,10 +202,10 @@ void launch_general(const ReplicaState* h_states, int count, ReplicaState* d_sta
                     int map_blocks = 0);
 // Replicas in which every group is a small rigid molecule moved by translate+rotate
 // (mc_rigid_kernel): whether a replica takes that route when it is not shared by several
-// workgroups, a function of the replica alone, and the launch of `count` such replicas.
+// workgroups, a function of the replica alone, and the launch of the replicas `ids`.
 bool rigid_route(const ReplicaState& s, bool f32);
-void launch_rigid(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
-                  TraceEntry* trace, int trace_cap, hipStream_t stream);
+void launch_rigid(const ReplicaState* h_states, const std::vector<int>& ids, const ReplicaMap& map, ReplicaState* d_states,
+                  const long long* d_moves, bool f32, TraceEntry* trace, int trace_cap, hipStream_t stream);
 // Fill a replica's fields for that route from its engine (after init or reset_positions).
 void set_rigid_fields(const Engine& e, ReplicaState& s, const std::vector<MoveKindSpec>& kinds);
 // Share a replica among `parts` workgroups of later general launches (1 undoes it);

@@ -305,7 +305,25 @@ __device__ __forceinline__ float pair_f32(const DevPairF& p, const CoulF& c, con
     }
 }
 
-// pair_energy_t of a form: the same arithmetic.
+// r = sqrt(r2) + 2^-52 (as the pair potentials form it) and 1 / r, from one reciprocal square
+// root by Newton steps: 12 FP64 operations where sqrt and a division take 50 instructions with
+// their scaling; r is the rounded root, 1 / r within an ulp.  Finite also for r2 = 0.
+__device__ __forceinline__ double distance(double r2, double& inv) {
+    const double x = r2 < 1e-30 ? 1e-30 : r2;
+    const double y = __builtin_amdgcn_rsq(x);
+    double r = x * y, h = 0.5 * y;
+    double e = fma(-h, r, 0.5);
+    r = fma(r, e, r);
+    h = fma(h, e, h);
+    r = fma(fma(-r, r, x), h, r);
+    r += 2.220446049250313e-16;
+    const double z = h + h;
+    inv = fma(z, fma(-r, z, 1.0), z);
+    inv = fma(inv, fma(-r, inv, 1.0), inv);
+    return r;
+}
+
+// pair_energy_t of a form: the same formulas.
 template <int kForm>
 __device__ __forceinline__ double pair_f64(const DevPair& p, const DevCoulomb& c, double qa, double qb, double r2,
                                            int terms) {
@@ -322,8 +340,9 @@ __device__ __forceinline__ double pair_f64(const DevPair& p, const DevCoulomb& c
         } else {
             u = (r2 < p.hs_s2) ? __builtin_huge_val() : 0.0;
         }
-        const double r = sqrt(r2) + 2.220446049250313e-16;
-        double e = c.lB * (qa * qb / r * coulomb_spline(c, r * c.rc_inv));
+        double inv;
+        const double r = distance(r2, inv);
+        double e = c.lB * (qa * qb * inv * coulomb_spline(c, r * c.rc_inv));
         materialize(e);
         return u + (r < c.rc && p.coul != 0.0 ? e : 0.0);
     }
@@ -336,16 +355,24 @@ template <class Fn> __device__ __forceinline__ void with_form(int form, Fn&& f) 
     else f(std::integral_constant<int, kFormAny>{});
 }
 
+// Whether particle j lies in the slots of this wave's lanes (uniform, scalar arithmetic).
+template <int kThreads, int kU> __device__ __forceinline__ bool moved_here(int j, int j0) {
+    const int d = j - __builtin_amdgcn_readfirstlane(j0);
+    return d >= 0 && d < kThreads * kU && (d & (kThreads - 1)) < 64;
+}
+
 // Pair sums of one moved particle, at its new (a) and old (b) position, against every
 // particle j in [jb, n) except `skip`; pairs inside group g count only if same_ok.
 // Lanes stride over j; each lane loads kU neighbours before evaluating them, whole waves
-// past the end excepted.  FP32 terms are summed in FP32 per block of kU and then in FP64; hot
+// past the end excepted; particle `moved` (-1: none), whose store may still be under way, is
+// taken at `at`.  FP32 terms are summed in FP32 per block of kU and then in FP64; hot
 // pairs go to the queue (hot_n, hot_q) with tag = moved atom << 1.
 template <int kThreads, int kForm>
 __device__ __forceinline__ void pair_row_f32(const FixPos* __restrict__ pos32, const uint32_t* __restrict__ meta, int jb,
                                              int n, int skip, int g, bool same_ok, const DevPairF* row, const CoulF& c,
                                              const float4* tab, int terms, float h, const FixPos& a, const FixPos& b,
-                                             int* hot_n, int2* hot_q, int tag, double& e_new, double& e_old) {
+                                             int* hot_n, int2* hot_q, int tag, double& e_new, double& e_old,
+                                             int moved = -1, const FixPos& at = FixPos{0u, 0u, 0u, 0.0f}) {
     constexpr int kU = 4;
     for (int j0 = jb + static_cast<int>(threadIdx.x); j0 < n; j0 += kThreads * kU) {
         FixPos pj[kU];
@@ -355,6 +382,11 @@ __device__ __forceinline__ void pair_row_f32(const FixPos* __restrict__ pos32, c
             const int j = min(j0 + u * kThreads, n - 1);
             pj[u] = pos32[j];
             mj[u] = meta[j];
+        }
+        if (moved_here<kThreads, kU>(moved, j0)) {
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (j0 + u * kThreads == moved) pj[u] = at;
         }
         float sn = 0.0f, so = 0.0f;
         bool anyhot = false;
@@ -414,7 +446,8 @@ __device__ __forceinline__ void pair_row_f64(const double4* __restrict__ pos, co
                                              int n, int skip, int g, bool same_ok, const DevPair* row,
                                              const DevCoulomb& c, int terms, const Box& box, double ax, double ay,
                                              double az, double bx, double by, double bz, double qa, double& e_new,
-                                             double& e_old) {
+                                             double& e_old, int moved = -1,
+                                             const double4& at = make_double4(0.0, 0.0, 0.0, 0.0)) {
     constexpr int kU = 2;
     for (int j0 = jb + static_cast<int>(threadIdx.x); j0 < n; j0 += kThreads * kU) {
         double4 pj[kU];
@@ -424,6 +457,11 @@ __device__ __forceinline__ void pair_row_f64(const double4* __restrict__ pos, co
             const int j = min(j0 + u * kThreads, n - 1);
             pj[u] = pos[j];
             mj[u] = meta[j];
+        }
+        if (moved_here<kThreads, kU>(moved, j0)) {
+#pragma unroll
+            for (int u = 0; u < kU; ++u)
+                if (j0 + u * kThreads == moved) pj[u] = at;
         }
         auto add = [&](int u) __attribute__((always_inline)) {
             const int j = j0 + u * kThreads;

@@ -202,10 +202,10 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
                                                                const long long* __restrict__ moves,
                                                                TraceEntry* __restrict__ trace, int trace_cap,
                                                                const int2* __restrict__ blockmap,
-                                                               long long spin_limit, int fix_lds) {
+                                                               long long spin_limit, int fix_lds, ReplicaMap map) {
     static_assert(!(kSplit && kCells), "the split form walks all particles");
     // block -> (replica, part); without split every block is part 0 of its own replica
-    const int2 bm = kSplit ? blockmap[blockIdx.x] : make_int2(static_cast<int>(blockIdx.x), 0);
+    const int2 bm = kSplit ? blockmap[blockIdx.x] : make_int2(map.first + map.id[blockIdx.x], 0);
     const int rep = bm.x, part = bm.y;
     if (kSplit && rep < 0) return; // an idle block of a placement map
     ReplicaState& S = states[rep];
@@ -1185,43 +1185,75 @@ __global__ void clear_general_slots_kernel(ReplicaState* __restrict__ states, in
     const int words = static_cast<int>(sizeof(GeneralSlot) / 8) * 2 * s.parts;
     for (int i = static_cast<int>(threadIdx.x); i < words; i += static_cast<int>(blockDim.x)) w[i] = 0ull;
 }
+// Dynamic LDS of a launch: the FP32 form keeps fixed-point copies of the moved atoms in LDS
+// where they fit (fix_lds).
+size_t general_lds(const GeneralLaunch& g, const void* fn, bool f32, int* fix_lds) {
+    const size_t limit = prepare(fn);
+    *fix_lds = f32 && g.lds + g.fix_lds_bytes <= limit ? 1 : 0;
+    const size_t lds = g.lds + (*fix_lds ? g.fix_lds_bytes : 0);
+    if (f32 && g.cells && !*fix_lds) throw std::runtime_error("molecules too large for the FP32 cell-list kernel's LDS");
+    if (lds > limit) throw std::runtime_error("k-vector and molecule tables too large for LDS");
+    return lds;
+}
+
+struct UnsplitLaunch {
+    const void* fn;
+    int threads, fix_lds;
+    size_t lds;
+};
+
+UnsplitLaunch plan_unsplit(const ReplicaState* h_states, const std::vector<int>& ids, bool f32) {
+    std::vector<ReplicaState> subset;
+    for (int r : ids) subset.push_back(h_states[r]);
+    const GeneralLaunch g = plan(subset.data(), static_cast<int>(subset.size()), f32);
+    UnsplitLaunch u{select_kernel(g.maxkpt, g.cells, f32, false), threads_of(g.cells), 0, 0};
+    u.lds = general_lds(g, u.fn, f32, &u.fix_lds);
+    return u;
+}
+
+// The replicas `ids` on mc_general_kernel, one workgroup each.
+void launch_unsplit(const ReplicaState* h_states, const std::vector<int>& ids, const ReplicaMap& map, ReplicaState* d_states,
+                    const long long* d_moves, bool f32, TraceEntry* trace, int trace_cap, hipStream_t stream) {
+    UnsplitLaunch u = plan_unsplit(h_states, ids, f32);
+    long long spin = 0;
+    const int2* none = nullptr;
+    ReplicaMap by_value = map;
+    void* args[] = {&d_states, &d_moves, &trace, &trace_cap, &none, &spin, &u.fix_lds, &by_value};
+    check_hip(hipLaunchKernel(u.fn, dim3(static_cast<unsigned>(ids.size())), dim3(u.threads), args, u.lds, stream),
+              "mc_general_kernel launch");
+}
+
 } // namespace
 
 void launch_general(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
                     TraceEntry* trace, int trace_cap, hipStream_t stream, const int2* d_blockmap, int map_blocks) {
-    // replicas of rigid molecules run their own kernel, in launches of their own (the route is
-    // a function of the replica alone); the server and Batch keep them apart from split ones
-    if (d_blockmap == nullptr) {
-        int r = 0;
-        while (r < count) {
-            int end = r;
-            const bool rigid = rigid_route(h_states[r], f32);
-            while (end < count && rigid_route(h_states[end], f32) == rigid) ++end;
-            if (!rigid && r == 0 && end == count) break; // all of them: below
-            TraceEntry* tr = trace ? trace + static_cast<size_t>(r) * trace_cap : nullptr;
-            if (rigid) launch_rigid(h_states + r, end - r, d_states + r, d_moves + r, f32, tr, trace_cap, stream);
-            else launch_general(h_states + r, end - r, d_states + r, d_moves + r, f32, tr, trace_cap, stream);
-            r = end;
-        }
-        if (r == count) return;
-    }
-    GeneralLaunch g = plan(h_states, count, f32);
-    const void* fn = select_kernel(g.maxkpt, g.cells, f32, g.split);
-    const size_t limit = prepare(fn);
-    // the FP32 form keeps fixed-point copies of the moved atoms in LDS where they fit
-    int fix_lds = f32 && g.lds + g.fix_lds_bytes <= limit ? 1 : 0;
-    if (fix_lds) g.lds += g.fix_lds_bytes;
-    if (f32 && g.cells && !fix_lds) throw std::runtime_error("molecules too large for the FP32 cell-list kernel's LDS");
-    if (g.lds > limit) throw std::runtime_error("k-vector and molecule tables too large for LDS");
-    // each workgroup lays out its own replica's tables inside the dynamic LDS
-    long long spin = 1LL << 24;
-    if (!g.split) {
-        const int2* none = nullptr;
-        void* args[] = {&d_states, &d_moves, &trace, &trace_cap, &none, &spin, &fix_lds};
-        check_hip(hipLaunchKernel(fn, dim3(count), dim3(threads_of(g.cells)), args, g.lds, stream),
-                  "mc_general_kernel launch");
+    // replicas that are not split run the kernel of their own route, one launch per route
+    bool split = false;
+    for (int r = 0; r < count; ++r) split = split || h_states[r].parts > 1;
+    if (!split) {
+        for (int r = 0; r < count; ++r) // as one launch of all of them was checked
+            if (h_states[r].cells != h_states[0].cells)
+                throw std::runtime_error("replicas of one launch must agree on the cell list");
+        const auto route = [&](int r) { return rigid_route(h_states[r], f32) ? 1 : 0; };
+        // every route's limits are checked before the first launch
+        launch_by_route(count, route, [&](const std::vector<int>& ids, const ReplicaMap&) {
+            if (!rigid_route(h_states[ids[0]], f32)) (void)plan_unsplit(h_states, ids, f32);
+        });
+        launch_by_route(count, route, [&](const std::vector<int>& ids, const ReplicaMap& map) {
+            if (rigid_route(h_states[ids[0]], f32))
+                launch_rigid(h_states, ids, map, d_states, d_moves, f32, trace, trace_cap, stream);
+            else
+                launch_unsplit(h_states, ids, map, d_states, d_moves, f32, trace, trace_cap, stream);
+        });
         return;
     }
+    const GeneralLaunch g = plan(h_states, count, f32);
+    const void* fn = select_kernel(g.maxkpt, g.cells, f32, g.split);
+    int fix_lds = 0;
+    const size_t lds = general_lds(g, fn, f32, &fix_lds);
+    // each workgroup lays out its own replica's tables inside the dynamic LDS
+    long long spin = 1LL << 24;
+    ReplicaMap none{};
     if (d_blockmap == nullptr) throw std::runtime_error("split general launch: block map missing");
     const int grid = map_blocks > 0 ? map_blocks : g.grid;
     if (grid < g.grid) throw std::runtime_error("split general launch: block map shorter than the parts");
@@ -1229,8 +1261,8 @@ void launch_general(const ReplicaState* h_states, int count, ReplicaState* d_sta
     static_assert(sizeof(GeneralSlot) % 8 == 0, "whole words");
     hipLaunchKernelGGL(clear_general_slots_kernel, dim3(count), dim3(64), 0, stream, d_states, count);
     check_hip(hipGetLastError(), "clear_general_slots_kernel");
-    void* args[] = {&d_states, &d_moves, &trace, &trace_cap, &d_blockmap, &spin, &fix_lds};
-    check_hip(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(kWide), args, static_cast<unsigned>(g.lds), stream),
+    void* args[] = {&d_states, &d_moves, &trace, &trace_cap, &d_blockmap, &spin, &fix_lds, &none};
+    check_hip(hipLaunchCooperativeKernel(fn, dim3(grid), dim3(kWide), args, static_cast<unsigned>(lds), stream),
               "mc_general_kernel cooperative launch");
 }
 

@@ -78,10 +78,12 @@ __host__ __device__ inline RigidLds rigid_lds(int ntypes, int ncut, int ngroups,
 template <int kEnt, bool kF32>
 __global__ __launch_bounds__(kRigidThreads) void mc_rigid_kernel(ReplicaState* __restrict__ states,
                                                                  const long long* __restrict__ moves,
-                                                                 TraceEntry* __restrict__ trace, int trace_cap) {
+                                                                 TraceEntry* __restrict__ trace, int trace_cap,
+                                                                 ReplicaMap map) {
     constexpr int kT = kRigidThreads;
-    ReplicaState& S = states[blockIdx.x];
-    const long long M = moves[blockIdx.x];
+    const int rep = map.first + map.id[blockIdx.x];
+    ReplicaState& S = states[rep];
+    const long long M = moves[rep];
     if (M <= 0 || S.error) return;
     __shared__ float4 s_stab[kF32 ? kSTable : 1];
     __shared__ DevCoulomb s_coul;
@@ -514,7 +516,7 @@ __global__ __launch_bounds__(kRigidThreads) void mc_rigid_kernel(ReplicaState* _
         }
         if (tid == 0) {
             if (trace && t < trace_cap) {
-                TraceEntry& T = trace[static_cast<size_t>(blockIdx.x) * trace_cap + t];
+                TraceEntry& T = trace[static_cast<size_t>(rep) * trace_cap + t];
                 T.index = m > 0 ? first : -1;
                 T.accepted = acc ? 1 : 0;
                 T.du = du;
@@ -596,7 +598,7 @@ __global__ __launch_bounds__(kRigidThreads) void mc_rigid_kernel(ReplicaState* _
     }
 }
 
-using RigidKernel = void (*)(ReplicaState*, const long long*, TraceEntry*, int);
+using RigidKernel = void (*)(ReplicaState*, const long long*, TraceEntry*, int, ReplicaMap);
 
 RigidKernel rigid_kernel(int entries, bool f32) {
     if (entries <= 2) return f32 ? mc_rigid_kernel<2, true> : mc_rigid_kernel<2, false>;
@@ -660,17 +662,17 @@ bool rigid_route(const ReplicaState& s, bool f32) {
     return s.rigid > 0 && s.parts <= 1 && rigid_bytes(s, f32) <= rigid_limit(rigid_entries(s), f32);
 }
 
-void launch_rigid(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
-                  TraceEntry* trace, int trace_cap, hipStream_t stream) {
+void launch_rigid(const ReplicaState* h_states, const std::vector<int>& ids, const ReplicaMap& map, ReplicaState* d_states,
+                  const long long* d_moves, bool f32, TraceEntry* trace, int trace_cap, hipStream_t stream) {
     int entries = 1;
     size_t lds = 0;
-    for (int r = 0; r < count; ++r) {
+    for (int r : ids) {
         entries = std::max(entries, rigid_entries(h_states[r]));
         lds = std::max(lds, rigid_bytes(h_states[r], f32));
     }
     (void)rigid_limit(entries, f32); // sets the kernels' attributes
-    hipLaunchKernelGGL(rigid_kernel(entries, f32), dim3(static_cast<unsigned>(count)), dim3(kRigidThreads), lds, stream,
-                       d_states, d_moves, trace, trace_cap);
+    hipLaunchKernelGGL(rigid_kernel(entries, f32), dim3(static_cast<unsigned>(ids.size())), dim3(kRigidThreads), lds, stream,
+                       d_states, d_moves, trace, trace_cap, map);
     check_hip(hipGetLastError(), "mc_rigid_kernel launch");
 }
 

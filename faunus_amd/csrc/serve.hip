@@ -177,10 +177,10 @@ void Server::step(long long quantum) {
     std::vector<int> order;
     // translate-only jobs also split by workgroup size (one launch each)
     auto launch_class = [&](const Slot& s) {
-        // (jobs of rigid molecules not split: 8, launches of their own)
+        // (8: jobs whose route takes another kernel, in launches of their own)
         return (s.state.cells != 0 ? 1 : 0) + (s.general ? 2 : 0) +
                (!s.general && advance_threads(s.state) == 512 ? 4 : 0) +
-               (s.general && s.parts == 1 && rigid_route(s.state, fp32_ != 0) ? 8 : 0);
+               ((s.general ? s.parts == 1 && rigid_route(s.state, fp32_ != 0) : translate_route(s.state)) ? 8 : 0);
     };
     // split jobs first within their class, so that they lead the cooperative launches
     for (int pass = 0; pass < 16; ++pass)
