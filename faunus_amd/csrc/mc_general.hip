@@ -32,7 +32,13 @@
 namespace fmc {
 namespace {
 
-constexpr int kChunk = 8;      // moved atoms per Ewald phase-table chunk
+constexpr int kChunk = 8;      // moved atoms per Ewald phase-table chunk of -ncut .. ncut (LDS)
+// Moved atoms from which the last particles of a slice (fewer than four per lane) are dealt
+// to the waves in columns of 64 (moved_column): with one particle per lane and step, 625
+// particles take two steps of which the second has 113 lanes at work.  A column's load is
+// repaid by a few moved atoms.  Chain of 350 beads in 10001 particles over 16 workgroups,
+// 1000 moves: 13.6 ms without columns, 12.7 ms with them.
+constexpr int kColumnAtoms = 8;
 constexpr int kMaxComb = 512;  // (moved atom, state, cell) combinations of the flattened stencil walk
 constexpr int kMaxParts = 64;  // workgroups per replica in the split form (one waiting lane each)
 constexpr int kMolStencil = 16; // moved atoms that may share one stencil (each member against all of them)
@@ -197,6 +203,77 @@ __device__ __forceinline__ void moved_block(int base, int je, const MovedSet& ms
     }
 }
 
+// Pair sums of the moved atoms [a0, a1) against one particle per lane, j (if j < je): the
+// particle sits in registers, the moved atoms stream from LDS two at a time, so that four
+// independent pair terms are in flight.  In the FP32 form each term is added in FP64, and a
+// hot pair goes to the queue in both states (a state at +inf, an overlap, keeps it).  Bound
+// by the pair terms' own instructions, about 60 each.
+template <bool kF32, bool kExcl, bool kCut, int kForm>
+__device__ __forceinline__ void moved_column(int j, int je, int a0, int a1, const MovedSet& ms,
+                                             const uint32_t* __restrict__ meta, const FixPos* __restrict__ pos32,
+                                             const double4* __restrict__ pos, const DevPairF* s_pairs_f,
+                                             const DevPair* s_pairs, int nt, const CoulF& cf, const float4* s_stab,
+                                             const DevCoulomb& s_coul, int terms, const Box& box, float hf, int* hot_n,
+                                             int2* hot_q, double& e_new, double& e_old) {
+    const bool in = j < je && !(j >= ms.mlo && j < ms.mhi);
+    const uint32_t mj = in ? meta[j] : 0u;
+    const int gj = static_cast<int>(mj >> 8), tj = static_cast<int>(mj & 0xffu);
+    const bool same = gj == ms.g;
+    const bool any = in && (!same || ms.same_ok);
+    if (!any) return;
+    const bool cut_n = kCut && !same && group_cut(ms.cut, gj, ms.cm_new, box);
+    const bool cut_o = kCut && !same && group_cut(ms.cut, gj, ms.cm_old, box);
+    FixPos pf{0u, 0u, 0u, 0.0f};
+    double4 pj = make_double4(0.0, 0.0, 0.0, 0.0);
+    if (kF32) pf = pos32[j];
+    else pj = pos[j];
+    for (int a = a0; a < a1; a += 2) {
+        float un[2], uo[2];
+        bool okn[2], oko[2], hot[2];
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const int av = min(a + v, a1 - 1);
+            const int ta = ms.s_mt[av];
+            const bool ok = a + v < a1 && !(kExcl && same && pair_excluded(ms.excl_off, ms.excl, ms.mlo + av, j));
+            okn[v] = ok && !cut_n;
+            oko[v] = ok && !cut_o;
+            if constexpr (kF32) {
+                const FixPos fa = ms.s_fnew[av], fb = ms.s_fold[av];
+                const DevPairF& p = s_pairs_f[ta * nt + tj];
+                bool hn, ho;
+                un[v] = pair_f32<kForm>(p, cf, s_stab, terms, fa.q, pf.q, dist2_fix(fa, pf, hf), hn);
+                uo[v] = pair_f32<kForm>(p, cf, s_stab, terms, fa.q, pf.q, dist2_fix(fb, pf, hf), ho);
+                hot[v] = (okn[v] && hn) || (oko[v] && ho);
+            } else {
+                const double4 A = ms.s_new[av], B = ms.s_old[av];
+                const DevPair& p = s_pairs[ta * nt + tj];
+                const double dn =
+                    pair_f64<kForm>(p, s_coul, A.w, pj.w, dist2(box, A.x, A.y, A.z, pj.x, pj.y, pj.z), terms);
+                const double dof =
+                    pair_f64<kForm>(p, s_coul, B.w, pj.w, dist2(box, B.x, B.y, B.z, pj.x, pj.y, pj.z), terms);
+                e_new += okn[v] ? dn : 0.0;
+                e_old += oko[v] ? dof : 0.0;
+            }
+        }
+        if constexpr (kF32) {
+            if (hot[0] || hot[1]) {
+#pragma unroll
+                for (int v = 0; v < 2; ++v) {
+                    if (!hot[v]) continue;
+                    if (okn[v] && un[v] != __builtin_huge_valf() && push_hot(hot_n, hot_q, j, (a + v) << 1)) okn[v] = false;
+                    if (oko[v] && uo[v] != __builtin_huge_valf() && push_hot(hot_n, hot_q, j, ((a + v) << 1) | 1))
+                        oko[v] = false;
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                e_new += okn[v] ? static_cast<double>(un[v]) : 0.0;
+                e_old += oko[v] ? static_cast<double>(uo[v]) : 0.0;
+            }
+        }
+    }
+}
+
 template <int kThreads, int kMaxKPT, bool kCells, bool kF32, bool kSplit>
 __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __restrict__ states,
                                                                const long long* __restrict__ moves,
@@ -237,7 +314,9 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
 
     const int tid = threadIdx.x;
     const int n = S.n, nk = S.nk, ncut = S.ncut, nt = S.ntypes;
-    const int width = 2 * ncut + 1;
+    const int w1 = ncut + 1; // phases of n = 0 .. ncut; those of -n are their conjugates
+    const int chunk = kChunk * (2 * ncut + 1) / w1; // atoms per phase-table chunk
+    const uint32_t w1_magic = (1u << 20) / static_cast<uint32_t>(w1) + 1u; // e / w1 for e * w1 < 2^20
     // this part's k-vectors [kb, ke) (kpt consecutive ones per thread) and static
     // particles [jb, je) of the pair sums
     const int kw = kSplit ? (nk + G - 1) / G : nk;
@@ -252,7 +331,7 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
     int* s_kn = s_dyn;
     double2* s_phase = reinterpret_cast<double2*>(s_dyn + nk8);
     const int max_moved = S.max_moved;
-    double4* s_nbuf = reinterpret_cast<double4*>(s_phase + kChunk * 6 * width);
+    double4* s_nbuf = reinterpret_cast<double4*>(s_phase + kChunk * 6 * (2 * ncut + 1));
     double4* s_old = s_nbuf + (kSplit ? 2 : 1) * max_moved;
     // fixed-point copies of the moved atoms for the FP32 pair paths when the launch's
     // LDS holds them (fix_lds); otherwise they are converted where they are used
@@ -289,6 +368,14 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
     const int form = pair_form(s_coul, S.terms, kF32);
 
     const int k0 = kb + tid * kpt;
+    // A part of few k-vectors leaves most threads without one (16 parts of 1000: 63 of 512), so
+    // the moved atoms are dealt to `segs` groups of kw threads, one k-vector per thread; the
+    // groups' sums meet in the phase tables' LDS after the last chunk (the case above: 14.9 ms
+    // with one group and tables of -ncut .. ncut, 13.6 ms)
+    const int nkp = max(ke - kb, 1);
+    const int segs = kpt == 1 ? max(1, min(kThreads / nkp, 1 + kChunk * 6 * (2 * ncut + 1) / nkp)) : 1;
+    const int seg = kpt == 1 ? tid / nkp : 0;
+    const int kseg = kb + (kpt == 1 ? tid % nkp : 0); // kpt == 1: this thread's k-vector
     double2 q[kMaxKPT];
 #pragma unroll
     for (int s = 0; s < kMaxKPT; ++s) q[s] = (s < kpt && k0 + s < ke) ? S.q[k0 + s] : make_double2(0.0, 0.0);
@@ -573,6 +660,23 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
                     int base = jb;
                     while (base < je) {
                         const int rem = je - base;
+                        if (m >= kColumnAtoms && rem < 4 * kThreads && (!kF32 || fixlds)) {
+                            // the last particles of the slice, 64 at a time, times the moved
+                            // atoms: (column, atom) pairs in equal runs over the waves
+                            const int work = ((rem + 63) >> 6) * m;
+                            constexpr int kWaves = kThreads / 64;
+                            const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+                            int lo = static_cast<int>(static_cast<long long>(work) * wave / kWaves);
+                            const int hi = static_cast<int>(static_cast<long long>(work) * (wave + 1) / kWaves);
+                            while (lo < hi) {
+                                const int col = lo / m, a0 = lo - col * m, a1 = min(m, a0 + hi - lo);
+                                moved_column<kF32, kX, kC, kP>(base + 64 * col + (tid & 63), je, a0, a1, ms, meta, pos32, pos,
+                                                               s_pairs_f, s_pairs, nt, cf, s_stab, s_coul, terms, box, hf,
+                                                               &s_nhot, s_hot, e_new, e_old);
+                                lo += a1 - a0;
+                            }
+                            break;
+                        }
                         if (kF32 && rem >= 8 * kThreads) {
                             moved_block<kThreads, 8, kF32, kX, kC, kP>(base, je, ms, meta, pos32, pos, s_pairs_f, s_pairs, nt, cf,
                                                                s_stab, s_coul, terms, box, hf, &s_nhot, s_hot, e_new, e_old);
@@ -778,38 +882,62 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
         double dqr[kMaxKPT], dqi[kMaxKPT];
 #pragma unroll
         for (int s = 0; s < kMaxKPT; ++s) dqr[s] = dqi[s] = 0.0;
-        for (int cst = 0; cst < m; cst += kChunk) {
-            const int cm_ = min(kChunk, m - cst);
-            if (cst > 0) __syncthreads(); // previous chunk's tables consumed
-            for (int e = tid; e < cm_ * 6 * width; e += kThreads) {
-                const int nn = e % width - ncut;
-                const int axis = (e / width) % 3;
-                const int st = (e / (3 * width)) & 1;
-                const int a = e / (6 * width);
-                const double4 A = st == 0 ? s_new[cst + a] : s_old[cst + a];
-                const double x = axis == 0 ? A.x : (axis == 1 ? A.y : A.z);
-                s_phase[e] = axis_phase(nn, x, inv);
+        for (int cst = 0; cst < m; cst += chunk) {
+            const int cm_ = min(chunk, m - cst);
+            if (cst > 0) lds_barrier(); // previous chunk's tables consumed
+            // from the last wave down: the first ones have more particles in the pair sums
+            for (int e = kThreads - 1 - tid; e < cm_ * 6 * w1; e += kThreads) {
+                const int row = static_cast<int>((static_cast<uint32_t>(e) * w1_magic) >> 20);
+                const int a = row / 6, c = row - 6 * a; // c: axis (new), 3 + axis (old)
+                const double* r = reinterpret_cast<const double*>((c < 3 ? s_new : s_old) + cst + a);
+                s_phase[e] = axis_phase(e - row * w1, r[c < 3 ? c : c - 3], inv);
             }
             __syncthreads();
+            // one atom's phase change at a k-vector
+            auto add_atom = [&](int a, int nx, int ny, int nz, double sy, double sz, double& xr, double& xi) {
+                const double2* tb = s_phase + a * 6 * w1;
+                const double2 xn = tb[nx], xo = tb[3 * w1 + nx];
+                double2 yn = tb[w1 + ny], zn = tb[2 * w1 + nz], yo = tb[4 * w1 + ny], zo = tb[5 * w1 + nz];
+                yn.y *= sy;
+                yo.y *= sy;
+                zn.y *= sz;
+                zo.y *= sz;
+                const double rn = xn.x * yn.x - xn.y * yn.y, in_ = xn.x * yn.y + xn.y * yn.x;
+                const double ro = xo.x * yo.x - xo.y * yo.y, io = xo.x * yo.y + xo.y * yo.x;
+                const double qa = s_new[cst + a].w;
+                xr += qa * ((rn * zn.x - in_ * zn.y) - (ro * zo.x - io * zo.y));
+                xi += qa * ((rn * zn.y + in_ * zn.x) - (ro * zo.y + io * zo.x));
+            };
+            if (kpt == 1) {
+                if (seg < segs && kseg < ke) {
+                    const int packed = s_kn[kseg];
+                    const int nx = unpack_n(packed, 0), ny = unpack_n(packed, 1), nz = unpack_n(packed, 2);
+                    for (int a = seg; a < cm_; a += segs)
+                        add_atom(a, nx, abs(ny), abs(nz), ny < 0 ? -1.0 : 1.0, nz < 0 ? -1.0 : 1.0, dqr[0], dqi[0]);
+                }
+            } else {
 #pragma unroll
-            for (int s = 0; s < kMaxKPT; ++s) {
-                const int k = k0 + s;
-                if (s < kpt && k < ke) {
-                    const int packed = s_kn[k];
-                    const int nx = unpack_n(packed, 0) + ncut, ny = unpack_n(packed, 1) + ncut,
-                              nz = unpack_n(packed, 2) + ncut;
-                    for (int a = 0; a < cm_; ++a) {
-                        const double2* tb = s_phase + a * 6 * width;
-                        const double2 xn = tb[nx], yn = tb[width + ny], zn = tb[2 * width + nz];
-                        const double2 xo = tb[3 * width + nx], yo = tb[4 * width + ny], zo = tb[5 * width + nz];
-                        const double rn = xn.x * yn.x - xn.y * yn.y, in_ = xn.x * yn.y + xn.y * yn.x;
-                        const double ro = xo.x * yo.x - xo.y * yo.y, io = xo.x * yo.y + xo.y * yo.x;
-                        const double qa = s_new[cst + a].w;
-                        dqr[s] += qa * ((rn * zn.x - in_ * zn.y) - (ro * zo.x - io * zo.y));
-                        dqi[s] += qa * ((rn * zn.y + in_ * zn.x) - (ro * zo.y + io * zo.x));
+                for (int s = 0; s < kMaxKPT; ++s) {
+                    const int k = k0 + s;
+                    if (s < kpt && k < ke) {
+                        const int packed = s_kn[k];
+                        const int nx = unpack_n(packed, 0), ny = unpack_n(packed, 1), nz = unpack_n(packed, 2);
+                        for (int a = 0; a < cm_; ++a)
+                            add_atom(a, nx, abs(ny), abs(nz), ny < 0 ? -1.0 : 1.0, nz < 0 ? -1.0 : 1.0, dqr[s], dqi[s]);
                     }
                 }
             }
+        }
+        if (segs > 1 && m > 1) { // uniform
+            lds_barrier();       // tables consumed
+            if (seg > 0 && seg < segs) s_phase[(seg - 1) * nkp + (kseg - kb)] = make_double2(dqr[0], dqi[0]);
+            lds_barrier();
+            if (seg == 0)
+                for (int g2 = 1; g2 < segs; ++g2) {
+                    const double2 v = s_phase[(g2 - 1) * nkp + tid];
+                    dqr[0] += v.x;
+                    dqi[0] += v.y;
+                }
         }
         if (kF32 && m > 0) {
             // hot pairs in FP64 from the FP64 coordinates (the Ewald chunk loop's barrier
