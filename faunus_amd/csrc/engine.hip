@@ -716,7 +716,7 @@ void Engine::upload_potentials() {
                 T.rmax2 = s.rmax2;
                 T.n = n;
                 T.hs = s.hardsphere ? 1 : 0;
-                std::fill(T.knots, T.knots + 2 * kSplMaxKnots, s.table.knots.back());
+                std::fill(T.knots, T.knots + kSplMaxKnots + 4, s.table.knots.back());
                 std::copy(s.table.knots.begin(), s.table.knots.end(), T.knots);
                 std::copy(s.table.coeff.begin(), s.table.coeff.end(), T.coeff);
                 T.x0 = s.table.knots.front();

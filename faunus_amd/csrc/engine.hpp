@@ -38,7 +38,7 @@ struct alignas(16) DevSplineTable {
     double rmin2, rmax2, x0, inv_w;
     int n, steps, hs, pad;
     double coeff[6 * kSplMaxKnots];
-    double knots[2 * kSplMaxKnots]; // padded with the last one past the search window
+    double knots[kSplMaxKnots + 4]; // padded with the last one past the search window
     unsigned char bucket[kSplBuckets + 16];
 };
 

@@ -274,6 +274,11 @@ __device__ __forceinline__ void moved_column(int j, int je, int a0, int a1, cons
     }
 }
 
+// Entries of the A_k table by |n|^2 = 0 .. ncut^2, rounded up to whole 16 bytes.  It lies in the
+// dynamic LDS at its own size: a table for ncut = 32 (8.2 KB) in the static LDS left molecules and
+// k-vector tables near the CU's limit without room (FP32: 77120 bytes, now 86928 less this table).
+__host__ __device__ __forceinline__ int gk_entries(int ncut) { return (ncut * ncut + 2) & ~1; }
+
 template <int kThreads, int kMaxKPT, bool kCells, bool kF32, bool kSplit>
 __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __restrict__ states,
                                                                const long long* __restrict__ moves,
@@ -293,7 +298,6 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
     __shared__ DevPairF s_pairs_f[kF32 ? kMaxTypes * kMaxTypes : 1];
     __shared__ float4 s_stab[kF32 ? kSTable : 1];
     __shared__ DevCoulomb s_coul;
-    __shared__ double s_gk[kMaxGk];
     __shared__ double s_dpa[kMaxTypes];
     __shared__ double s_mw[kMaxTypes];          // atom masses (cutoff_g2g mass centres)
     __shared__ double s_cm[2][3];               // the moved group's mass centre, new and old state
@@ -310,7 +314,7 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
     __shared__ MoveDraw s_draw[kDraw];
     // kn | phase chunk tables | new coordinates (two buffers in the split form) | old
     // coordinates | (FP32 form) fixed-point new and old coordinates | moved types
-    extern __shared__ int s_dyn[];
+    extern __shared__ __align__(16) int s_dyn[];
 
     const int tid = threadIdx.x;
     const int n = S.n, nk = S.nk, ncut = S.ncut, nt = S.ntypes;
@@ -328,8 +332,9 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
     const int je = kSplit ? min(n, jb + jw) : n;
     const double L = S.L, half = S.half, inv = S.inv;
     const int nk8 = (nk + 7) & ~7;
-    int* s_kn = s_dyn;
-    double2* s_phase = reinterpret_cast<double2*>(s_dyn + nk8);
+    double* s_gk = reinterpret_cast<double*>(s_dyn); // A_k by |n|^2
+    int* s_kn = reinterpret_cast<int*>(s_gk + gk_entries(ncut));
+    double2* s_phase = reinterpret_cast<double2*>(s_kn + nk8);
     const int max_moved = S.max_moved;
     double4* s_nbuf = reinterpret_cast<double4*>(s_phase + kChunk * 6 * (2 * ncut + 1));
     double4* s_old = s_nbuf + (kSplit ? 2 : 1) * max_moved;
@@ -357,7 +362,7 @@ __global__ __launch_bounds__(kThreads) void mc_general_kernel(ReplicaState* __re
         s_mw[i] = S.mw != nullptr ? S.mw[i] : 1.0;
     }
     for (int i = tid; i < S.nkinds; i += kThreads) s_kinds[i] = S.kinds[i];
-    for (int i = tid; i <= ncut * ncut && i < kMaxGk; i += kThreads) s_gk[i] = S.gk[i];
+    for (int i = tid; i <= ncut * ncut; i += kThreads) s_gk[i] = S.gk[i];
     for (int k = tid; k < nk; k += kThreads) s_kn[k] = S.kn[k];
     __syncthreads();
     if (kF32) {
@@ -1197,15 +1202,17 @@ const void* select_kernel(int maxkpt, bool cells, bool f32, bool split) {
 
 constexpr size_t kLdsPerCU = 160 * 1024;
 
-// Dynamic LDS a kernel may take: what its static LDS leaves of the CU's 160 KB, at
-// most 96 KB (set once per kernel).
+constexpr size_t kMaxTables = 96 * 1024; // dynamic LDS without the A_k table
+
+// Dynamic LDS a kernel may take: what its static LDS leaves of the CU's 160 KB (set once per
+// kernel), at most kMaxTables and the largest A_k table.
 size_t prepare(const void* fn) {
     static std::vector<std::pair<const void*, size_t>> done;
     for (const auto& d : done)
         if (d.first == fn) return d.second;
     hipFuncAttributes attr;
     check_hip(hipFuncGetAttributes(&attr, fn), "hipFuncGetAttributes");
-    const size_t limit = std::min<size_t>(96 * 1024, kLdsPerCU - attr.sharedSizeBytes);
+    const size_t limit = std::min(kMaxTables + sizeof(double) * (kMaxGk + 1), kLdsPerCU - attr.sharedSizeBytes);
     check_hip(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(limit)),
               "hipFuncSetAttribute");
     done.emplace_back(fn, limit);
@@ -1226,10 +1233,11 @@ struct GeneralLaunch {
     size_t lds;
     int grid;
     size_t fix_lds_bytes; // FP32 form: fixed-point copies of the moved atoms
+    size_t gk_bytes;      // A_k table, part of lds
 };
 
 GeneralLaunch plan(const ReplicaState* h_states, int count, bool f32) {
-    GeneralLaunch g{0, h_states[0].cells != 0, false, 0, 0};
+    GeneralLaunch g{0, h_states[0].cells != 0, false, 0, 0, 0, 0};
     int maxnk = 0, maxw = 0, maxm = 0;
     for (int r = 0; r < count; ++r) {
         const ReplicaState& s = h_states[r];
@@ -1251,7 +1259,8 @@ GeneralLaunch plan(const ReplicaState* h_states, int count, bool f32) {
     if (g.maxkpt > kpt_cap(g.cells))
         throw std::runtime_error("too many k-vectors for the general device MC (max 4096 per workgroup)");
     // the split form keeps the previous move's coordinates in a second buffer
-    g.lds = sizeof(int) * static_cast<size_t>((maxnk + 7) & ~7) + sizeof(double2) * kChunk * 6 * static_cast<size_t>(maxw) +
+    g.gk_bytes = sizeof(double) * static_cast<size_t>(gk_entries((maxw - 1) / 2));
+    g.lds = g.gk_bytes + sizeof(int) * static_cast<size_t>((maxnk + 7) & ~7) + sizeof(double2) * kChunk * 6 * static_cast<size_t>(maxw) +
             ((g.split ? 3 : 2) * sizeof(double4) + sizeof(int)) * static_cast<size_t>(maxm);
     g.fix_lds_bytes = 2 * sizeof(FixPos) * static_cast<size_t>(maxm);
     return g;
@@ -1316,7 +1325,7 @@ __global__ void clear_general_slots_kernel(ReplicaState* __restrict__ states, in
 // Dynamic LDS of a launch: the FP32 form keeps fixed-point copies of the moved atoms in LDS
 // where they fit (fix_lds).
 size_t general_lds(const GeneralLaunch& g, const void* fn, bool f32, int* fix_lds) {
-    const size_t limit = prepare(fn);
+    const size_t limit = std::min(prepare(fn), kMaxTables + g.gk_bytes);
     *fix_lds = f32 && g.lds + g.fix_lds_bytes <= limit ? 1 : 0;
     const size_t lds = g.lds + (*fix_lds ? g.fix_lds_bytes : 0);
     if (f32 && g.cells && !*fix_lds) throw std::runtime_error("molecules too large for the FP32 cell-list kernel's LDS");
