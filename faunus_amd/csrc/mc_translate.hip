@@ -40,8 +40,11 @@ struct TranslateTotals {
     unsigned long long accepted, e_samples;
 };
 
+// Two waves per SIMD, so at most 256 VGPRs: with 256 threads two workgroups share a CU, whose
+// 160 KB of LDS hold both also in the FP32 form (73.2 KB static and at most 8 KB of k-vectors each;
+// with 512 threads, one per CU, A_k is staged in 8 KB more for the set-up).
 template <int kThreads, int kEnt, bool kCells, bool kF32>
-__global__ __launch_bounds__(kThreads) void mc_translate_kernel(ReplicaState* __restrict__ states,
+__global__ __launch_bounds__(kThreads, 2) void mc_translate_kernel(ReplicaState* __restrict__ states,
                                                                 const long long* __restrict__ moves,
                                                                 TraceEntry* __restrict__ trace, int trace_cap,
                                                                 const LadderRun* __restrict__ ladders, ReplicaMap map) {
@@ -58,7 +61,7 @@ __global__ __launch_bounds__(kThreads) void mc_translate_kernel(ReplicaState* __
     __shared__ float4 s_stab[kF32 ? kSTable : 1];
     __shared__ DevCoulomb s_coul;
     __shared__ double s_dp[kMaxTypes];
-    __shared__ double s_gk[kMaxGk];
+    __shared__ double s_gk[kThreads > 256 ? kMaxGk : 1];
     __shared__ double s_red[3][kWaves];
     __shared__ int s_scan[kWaves];
     __shared__ int s_nhot[2]; // hot pairs queued (FP32 form), by move parity
@@ -80,7 +83,8 @@ __global__ __launch_bounds__(kThreads) void mc_translate_kernel(ReplicaState* __
     }
     lds_copy(s_coul, S.coul, tid, kThreads);
     for (int i = tid; i < nt; i += kThreads) s_dp[i] = S.dp_type[i];
-    for (int i = tid; i <= ncut * ncut && i < kMaxGk; i += kThreads) s_gk[i] = S.gk[i];
+    if (kThreads > 256)
+        for (int i = tid; i <= ncut * ncut && i < kMaxGk; i += kThreads) s_gk[i] = S.gk[i];
     if (kF32 && S.stab)
         for (int i = tid; i < kSTable; i += kThreads) s_stab[i] = S.stab[i];
     if (tid == 0) {
@@ -117,7 +121,8 @@ __global__ __launch_bounds__(kThreads) void mc_translate_kernel(ReplicaState* __
             nx[s] = unpack_n(packed, 0);
             ny[s] = unpack_n(packed, 1);
             nz[s] = unpack_n(packed, 2);
-            ak[s] = (nx[s] > 0 ? 2.0 : 1.0) * s_gk[nx[s] * nx[s] + ny[s] * ny[s] + nz[s] * nz[s]];
+            const int n2 = nx[s] * nx[s] + ny[s] * ny[s] + nz[s] * nz[s];
+            ak[s] = (nx[s] > 0 ? 2.0 : 1.0) * (kThreads > 256 ? s_gk[n2] : S.gk[n2]);
             qp[s] = S.q[kp[s]];
             if (nz[s] > 0) qm[s] = S.q[kp[s] - 2 * nz[s] + (nx[s] == 0 && ny[s] == 0 ? 1 : 0)];
             if (ny[s] < 0) {
