@@ -88,6 +88,36 @@ Batch::Batch(int precision_fp32) : fp32_(precision_fp32) {
     check_hip(hipEventCreate(&ev1_), "hipEventCreate");
 }
 
+SideBySide::~SideBySide() {
+    for (int k = 0; k < kStreams; ++k) {
+        if (streams_[k]) (void)hipStreamDestroy(streams_[k]);
+        if (done_[k]) (void)hipEventDestroy(done_[k]);
+    }
+    if (forked_) (void)hipEventDestroy(forked_);
+}
+
+// The first `side` streams wait for all that was enqueued on `main`.
+void SideBySide::fork(hipStream_t main, int side) {
+    if (!forked_) check_hip(hipEventCreateWithFlags(&forked_, hipEventDisableTiming), "hipEventCreate");
+    for (int k = 0; k < side; ++k) {
+        if (!streams_[k]) check_hip(hipStreamCreateWithFlags(&streams_[k], hipStreamNonBlocking), "hipStreamCreate");
+        if (!done_[k]) check_hip(hipEventCreateWithFlags(&done_[k], hipEventDisableTiming), "hipEventCreate");
+    }
+    check_hip(hipEventRecord(forked_, main), "fork streams");
+    for (int k = 0; k < side; ++k) check_hip(hipStreamWaitEvent(streams_[k], forked_, 0), "fork streams");
+}
+
+// `main` waits for them; the first error, after all have been joined as far as possible.
+hipError_t SideBySide::join(hipStream_t main, int side) {
+    hipError_t first = hipSuccess;
+    for (int k = 0; k < side; ++k) {
+        hipError_t e = hipEventRecord(done_[k], streams_[k]);
+        if (e == hipSuccess) e = hipStreamWaitEvent(main, done_[k], 0);
+        if (first == hipSuccess) first = e;
+    }
+    return first;
+}
+
 Batch::~Batch() {
     if (stream_) (void)hipStreamSynchronize(stream_);
     if (graph_) (void)hipGraphExecDestroy(graph_);
@@ -420,7 +450,7 @@ int advance_threads(const ReplicaState& s) {
 }
 
 void launch_advance(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
-                    TraceEntry* trace, int trace_cap, hipStream_t stream, const LadderRun* ladders) {
+                    TraceEntry* trace, int trace_cap, hipStream_t stream, SideBySide& side, const LadderRun* ladders) {
     // workgroup size and kernel of each replica, functions of the replica alone (so that its
     // arithmetic does not depend on its batch), except that the replicas of a ladder launch
     // with cell lists take 256 threads, and the kernel for any K, when they do not agree
@@ -457,20 +487,20 @@ void launch_advance(const ReplicaState* h_states, int count, ReplicaState* d_sta
     };
     for (int r = 0; r < count; ++r)
         if (table_bytes({r}) > 96 * 1024) throw std::runtime_error("k-vector table too large for LDS");
-    launch_by_route(count, [&](int r) { return 2 * threads[static_cast<size_t>(r)] + translate[static_cast<size_t>(r)]; },
-                    [&](const std::vector<int>& ids, const ReplicaMap& map) {
-        const size_t first = static_cast<size_t>(ids[0]);
+    const auto route = [&](int r) { return 2 * threads[static_cast<size_t>(r)] + translate[static_cast<size_t>(r)]; };
+    side.run(launches_by_route(count, route), stream, [&](const RouteLaunch& l, hipStream_t on) {
+        const size_t first = static_cast<size_t>(l.ids[0]);
         if (translate[first]) {
-            launch_translate(h_states, ids, map, threads[first], d_states, d_moves, f32, trace, trace_cap, stream, ladders);
+            launch_translate(h_states, l.ids, l.map, threads[first], d_states, d_moves, f32, trace, trace_cap, on, ladders);
             return;
         }
         int kpt = 0;
-        for (int r : ids) kpt = std::max(kpt, (h_states[r].nk + 255) / 256);
-        const int grid = static_cast<int>(ids.size());
-        const size_t lds = table_bytes(ids);
-        const auto go = [&](auto launch) { launch(grid, lds, stream, d_states, d_moves, trace, trace_cap, ladders, map); };
+        for (int r : l.ids) kpt = std::max(kpt, (h_states[r].nk + 255) / 256);
+        const int grid = static_cast<int>(l.ids.size());
+        const size_t lds = table_bytes(l.ids);
+        const auto go = [&](auto launch) { launch(grid, lds, on, d_states, d_moves, trace, trace_cap, ladders, l.map); };
         if (kpt > 32 && (cells || !f32))
-            launch_wide(cells, f32, grid, lds, stream, d_states, d_moves, trace, trace_cap, ladders, map);
+            launch_wide(cells, f32, grid, lds, on, d_states, d_moves, trace, trace_cap, ladders, l.map);
         else if (kpt > 32) go(launch_advance<68, false, true>);
         else if (cells) go(f32 ? launch_advance<32, true, true> : launch_advance<32, true, false>);
         else go(f32 ? launch_advance<32, false, true> : launch_advance<32, false, false>);
@@ -566,9 +596,9 @@ void Batch::run(const std::vector<long long>& moves, bool trace, int trace_cap) 
         // one workgroup per replica, also for replicas that earlier ran split
         std::vector<ReplicaState> one(h_states_);
         for (auto& s : one) s.parts = 1;
-        launch_general(one.data(), size(), d_states_, d_moves_, fp32_ != 0, tr, cap, stream_);
+        launch_general(one.data(), size(), d_states_, d_moves_, fp32_ != 0, tr, cap, stream_, side_);
     }
-    else launch_advance(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, tr, cap, stream_);
+    else launch_advance(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, tr, cap, stream_, side_);
     time_end();
 }
 
@@ -824,15 +854,15 @@ void Batch::capture_interval(const std::vector<long long>& moves, unsigned long 
     // one launch outside the capture sets the kernels' attributes (not a stream operation)
     const std::vector<long long> zero(static_cast<size_t>(size()), 0);
     check_hip(hipMemcpy(d_moves_, zero.data(), sizeof(long long) * size(), hipMemcpyHostToDevice), "copy moves");
-    if (general_ == 1) launch_general(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_);
-    else launch_advance(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_);
+    if (general_ == 1) launch_general(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_, side_);
+    else launch_advance(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_, side_);
     check_hip(hipStreamSynchronize(stream_), "attribute run");
     check_hip(hipMemcpy(d_moves_, moves.data(), sizeof(long long) * size(), hipMemcpyHostToDevice), "copy moves");
     hipGraph_t g = nullptr;
     check_hip(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     try {
-        if (general_ == 1) launch_general(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_);
-        else launch_advance(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_);
+        if (general_ == 1) launch_general(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_, side_);
+        else launch_advance(h_states_.data(), size(), d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_, side_);
         if (nl > 0) {
             hipLaunchKernelGGL(ladder_swap_kernel, dim3(1), dim3(((nl + 63) / 64) * 64), 0, stream_, d_states_, d_lb, d_ls,
                                d_rung, nl, seed, 0ull, d_cnt, d_cnt + 2);
@@ -928,7 +958,7 @@ void Batch::run_ladders(const std::vector<long long>& moves, const std::vector<i
         check_hip(hipMemcpy(d_moves_, moves.data(), sizeof(long long) * n, hipMemcpyHostToDevice), "copy moves");
         check_hip(hipMemcpy(d, host.data(), bytes, hipMemcpyHostToDevice), "copy ladders");
         time_begin();
-        launch_advance(h_states_.data(), n, d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_,
+        launch_advance(h_states_.data(), n, d_states_, d_moves_, fp32_ != 0, nullptr, 0, stream_, side_,
                        reinterpret_cast<const LadderRun*>(d));
         time_end();
         unsigned long long cnt[2] = {0, 0};

@@ -1363,8 +1363,9 @@ void launch_unsplit(const ReplicaState* h_states, const std::vector<int>& ids, c
 } // namespace
 
 void launch_general(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
-                    TraceEntry* trace, int trace_cap, hipStream_t stream, const int2* d_blockmap, int map_blocks) {
-    // replicas that are not split run the kernel of their own route, one launch per route
+                    TraceEntry* trace, int trace_cap, hipStream_t stream, SideBySide& side, const int2* d_blockmap,
+                    int map_blocks) {
+    // replicas that are not split run the kernel of their own route, one launch per route, side by side
     bool split = false;
     for (int r = 0; r < count; ++r) split = split || h_states[r].parts > 1;
     if (!split) {
@@ -1372,15 +1373,15 @@ void launch_general(const ReplicaState* h_states, int count, ReplicaState* d_sta
             if (h_states[r].cells != h_states[0].cells)
                 throw std::runtime_error("replicas of one launch must agree on the cell list");
         const auto route = [&](int r) { return rigid_route(h_states[r], f32) ? 1 : 0; };
+        const std::vector<RouteLaunch> launches = launches_by_route(count, route);
         // every route's limits are checked before the first launch
-        launch_by_route(count, route, [&](const std::vector<int>& ids, const ReplicaMap&) {
-            if (!rigid_route(h_states[ids[0]], f32)) (void)plan_unsplit(h_states, ids, f32);
-        });
-        launch_by_route(count, route, [&](const std::vector<int>& ids, const ReplicaMap& map) {
-            if (rigid_route(h_states[ids[0]], f32))
-                launch_rigid(h_states, ids, map, d_states, d_moves, f32, trace, trace_cap, stream);
+        for (const RouteLaunch& l : launches)
+            if (!rigid_route(h_states[l.ids[0]], f32)) (void)plan_unsplit(h_states, l.ids, f32);
+        side.run(launches, stream, [&](const RouteLaunch& l, hipStream_t on) {
+            if (rigid_route(h_states[l.ids[0]], f32))
+                launch_rigid(h_states, l.ids, l.map, d_states, d_moves, f32, trace, trace_cap, on);
             else
-                launch_unsplit(h_states, ids, map, d_states, d_moves, f32, trace, trace_cap, stream);
+                launch_unsplit(h_states, l.ids, l.map, d_states, d_moves, f32, trace, trace_cap, on);
         });
         return;
     }

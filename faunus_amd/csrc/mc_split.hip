@@ -1241,7 +1241,7 @@ void Batch::run_split_general(long long moves, int groups, int stride, bool trac
     check_hip(hipMemcpyAsync(d_moves_, &h_split_moves_, sizeof(long long), hipMemcpyHostToDevice, stream_), "copy moves");
     time_begin();
     launch_general(h_states_.data(), 1, d_states_, d_moves_, fp32_ != 0, trace ? d_trace_ : nullptr,
-                   trace ? trace_cap : 0, stream_, groups > 1 ? d_map_ : nullptr, groups > 1 ? grid : 0);
+                   trace ? trace_cap : 0, stream_, side_, groups > 1 ? d_map_ : nullptr, groups > 1 ? grid : 0);
     time_end();
 }
 

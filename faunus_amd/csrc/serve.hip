@@ -175,19 +175,17 @@ void Server::step(long long quantum) {
     std::vector<ReplicaState> states(static_cast<size_t>(count));
     std::vector<long long> moves(static_cast<size_t>(count));
     std::vector<int> order;
-    // translate-only jobs also split by workgroup size (one launch each)
-    auto launch_class = [&](const Slot& s) {
-        // (8: jobs whose route takes another kernel, in launches of their own)
-        return (s.state.cells != 0 ? 1 : 0) + (s.general ? 2 : 0) +
-               (!s.general && advance_threads(s.state) == 512 ? 4 : 0) +
-               ((s.general ? s.parts == 1 && rigid_route(s.state, fp32_ != 0) : translate_route(s.state)) ? 8 : 0);
+    auto launch_class = [&](const Slot& s) { return (s.state.cells != 0 ? 1 : 0) + (s.general ? 2 : 0); };
+    // within a class split jobs first, so that they lead the cooperative launches, and jobs of
+    // rigid molecules last, whose kernel those launches do not run
+    auto rank = [&](const Slot& s) {
+        return s.parts > 1 ? 0 : (s.general && rigid_route(s.state, fp32_ != 0) ? 2 : 1);
     };
-    // split jobs first within their class, so that they lead the cooperative launches
-    for (int pass = 0; pass < 16; ++pass)
-        for (int split = 1; split >= 0; --split)
+    for (int pass = 0; pass < 4; ++pass)
+        for (int want = 0; want < 3; ++want)
             for (int k = 0; k < count; ++k) {
                 const Slot& s = active_[static_cast<size_t>(k)];
-                if (launch_class(s) == pass && (s.parts > 1 ? 1 : 0) == split) order.push_back(k);
+                if (launch_class(s) == pass && rank(s) == want) order.push_back(k);
             }
     for (int r = 0; r < count; ++r) {
         const Slot& s = active_[static_cast<size_t>(order[static_cast<size_t>(r)])];
@@ -222,7 +220,7 @@ void Server::step(long long quantum) {
                 int blocks = 0;
                 while (b < last) {
                     const int p = std::max(1, states[static_cast<size_t>(b)].parts);
-                    if (blocks + p > coresident_) break;
+                    if (blocks + p > coresident_ || rigid_route(states[static_cast<size_t>(b)], fp32_ != 0)) break;
                     blocks += p;
                     ++b;
                 }
@@ -251,10 +249,10 @@ void Server::step(long long quantum) {
     for (const Launch& l : launches) {
         if (l.cls & 2)
             launch_general(states.data() + l.first, l.last - l.first, d_states_ + l.first, d_moves_ + l.first,
-                           fp32_ != 0, nullptr, 0, stream_, l.map_off >= 0 ? d_map_ + l.map_off : nullptr);
+                           fp32_ != 0, nullptr, 0, stream_, side_, l.map_off >= 0 ? d_map_ + l.map_off : nullptr);
         else
             launch_advance(states.data() + l.first, l.last - l.first, d_states_ + l.first, d_moves_ + l.first,
-                           fp32_ != 0, nullptr, 0, stream_);
+                           fp32_ != 0, nullptr, 0, stream_, side_);
     }
     check_hip(hipMemcpyAsync(states.data(), d_states_, sizeof(ReplicaState) * count, hipMemcpyDeviceToHost, stream_),
               "copy states back");

@@ -78,6 +78,7 @@ class Server {
     size_t used_ = 0;
     long long moves_total_ = 0;
     hipStream_t stream_ = nullptr;
+    SideBySide side_;
     ReplicaState* d_states_ = nullptr;
     long long* d_moves_ = nullptr;
     int capacity_ = 0;
