@@ -306,10 +306,11 @@ __device__ __forceinline__ float pair_f32(const DevPairF& p, const CoulF& c, con
 }
 
 // r = sqrt(r2) + 2^-52 (as the pair potentials form it) and 1 / r, from one reciprocal square
-// root by Newton steps: 12 FP64 operations where sqrt and a division take 50 instructions with
-// their scaling; r is the rounded root, 1 / r within an ulp.  Finite also for r2 = 0.
+// root and one reciprocal by Newton steps: 13 FP64 operations where sqrt and a division take 50
+// instructions with their scaling; r is the rounded root, 1 / r within an ulp.  Finite also for
+// r2 = 0, where r is 2^-52.
 __device__ __forceinline__ double distance(double r2, double& inv) {
-    const double x = r2 < 1e-30 ? 1e-30 : r2;
+    const double x = r2 < 1e-280 ? 1e-280 : r2;
     const double y = __builtin_amdgcn_rsq(x);
     double r = x * y, h = 0.5 * y;
     double e = fma(-h, r, 0.5);
@@ -317,8 +318,8 @@ __device__ __forceinline__ double distance(double r2, double& inv) {
     h = fma(h, e, h);
     r = fma(fma(-r, r, x), h, r);
     r += 2.220446049250313e-16;
-    const double z = h + h;
-    inv = fma(z, fma(-r, z, 1.0), z);
+    inv = __builtin_amdgcn_rcp(r); // 2 h would be the reciprocal before the addition
+    inv = fma(inv, fma(-r, inv, 1.0), inv);
     inv = fma(inv, fma(-r, inv, 1.0), inv);
     return r;
 }
