@@ -39,6 +39,8 @@ __global__ void ladder_swap_kernel(ReplicaState* states, const int* ladder_begin
     swap_ladder_rungs(states, ladder_begin[l], ladder_size[l], rung_slot, l, seed, round, counters);
 }
 
+constexpr int kRdfList = 2048;
+
 // Pair-distance histogram of one configuration (AtomRDF::_sample, analysis.cpp:1556-1600):
 // types a != b: every (a, b) pair; a == b: pairs i < j.  r = |minimum-image distance|,
 // bin floor(r / dr) as Equidistant2DTable::to_bin (equidistant_table.h:32-39), bins >= nbins
@@ -46,8 +48,11 @@ __global__ void ladder_swap_kernel(ReplicaState* states, const int* ladder_begin
 // them), against the i of type a in run y of `len` particles, whose coordinates are the
 // same for every lane (scalar loads).  Pairs beyond the last bin (range2: 1e-9 above its
 // squared edge) stop at the rounded distance; counts go to an LDS histogram, then once
-// per block to the global one.  N = 20000, 240 bins of 0.1 A: 717 us with one i per block
+// per block to the global one.  Up to kRdfList particles, where the
+// list's copy to the device takes longer than the lanes it saves, every particle has a thread
+// (kList false): N = 200 37 -> 29 us a call, N = 4000 74 us against 59 with the list.  N = 20000, 240 bins of 0.1 A: 717 us with one i per block
 // (every block read all positions), now 125 us.
+template <bool kList>
 __global__ __launch_bounds__(256) void rdf_kernel(const double4* __restrict__ pos, const uint32_t* __restrict__ meta,
                                                   int n, int ta, int tb, double L, double half, double inv_dr,
                                                   double range2, int nbins, int len, const int* __restrict__ ids, int nb,
@@ -55,7 +60,8 @@ __global__ __launch_bounds__(256) void rdf_kernel(const double4* __restrict__ po
     extern __shared__ unsigned int s_hist[];
     for (int b = threadIdx.x; b < nbins; b += blockDim.x) s_hist[b] = 0u;
     const int t = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    const int j = t < nb ? ids[t] : -1;
+    int j = -1;
+    if (t < nb) j = kList ? ids[t] : (static_cast<int>(meta[t] & 0xffu) == tb ? t : -1);
     const double4 pj = pos[max(j, 0)];
     const Box box{{L, L, L}, {half, half, half}};
     const double inv[3] = {1.0 / L, 1.0 / L, 1.0 / L};
@@ -631,22 +637,26 @@ void Batch::rdf(int r, int type_a, int type_b, double dr, int nbins, unsigned lo
     for (int j = 0; j < h.n; ++j)
         if (types[static_cast<size_t>(j)] == type_b) ids.push_back(j);
     if (ids.empty()) return;
-    const int nb = static_cast<int>(ids.size());
+    if (h.n <= kRdfList) ids.clear();
+    const int nb = ids.empty() ? h.n : static_cast<int>(ids.size());
     const size_t head = (sizeof(int) * ids.size() + 7) & ~static_cast<size_t>(7);
     unsigned char* d = nullptr;
     check_hip(hipMalloc(&d, head + sizeof(unsigned long long) * static_cast<size_t>(nbins)), "hipMalloc rdf");
     unsigned long long* d_counts = reinterpret_cast<unsigned long long*>(d + head);
     std::vector<unsigned long long> part(static_cast<size_t>(nbins));
     try {
-        check_hip(hipMemcpyAsync(d, ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice, stream_), "copy rdf ids");
+        if (!ids.empty())
+            check_hip(hipMemcpyAsync(d, ids.data(), sizeof(int) * ids.size(), hipMemcpyHostToDevice, stream_), "copy rdf ids");
         check_hip(hipMemsetAsync(d_counts, 0, sizeof(unsigned long long) * static_cast<size_t>(nbins), stream_),
                   "clear rdf");
         const int tiles = (nb + 255) / 256;
-        // about 2048 blocks, each with at least 32 i for its histogram's clear and flush
-        const int runs = std::max(1, std::min((h.n + 31) / 32, 2048 / tiles));
+        // about 2048 blocks, each with at least 32 i for its histogram's clear and flush (fewer,
+        // down to 4, where that leaves CUs without a block)
+        const int least = std::max(4, std::min(32, static_cast<int>(static_cast<long long>(h.n) * tiles / 256)));
+        const int runs = std::max(1, std::min((h.n + least - 1) / least, 2048 / tiles));
         const int len = (h.n + runs - 1) / runs;
         const double edge = static_cast<double>(nbins) * dr;
-        hipLaunchKernelGGL(rdf_kernel, dim3(static_cast<unsigned>(tiles), static_cast<unsigned>((h.n + len - 1) / len)),
+        hipLaunchKernelGGL(ids.empty() ? rdf_kernel<false> : rdf_kernel<true>, dim3(static_cast<unsigned>(tiles), static_cast<unsigned>((h.n + len - 1) / len)),
                            dim3(256), sizeof(unsigned int) * static_cast<size_t>(nbins), stream_, h.pos, h.meta, h.n, type_a,
                            type_b, h.L, h.half, 1.0 / dr, edge * edge * (1.0 + 1e-9), nbins, len,
                            reinterpret_cast<const int*>(d), nb, d_counts);
