@@ -67,6 +67,7 @@ SIGNATURES = {
     "fmc_batch_set_timing": (C.c_int, [C.c_void_p, C.c_int]),
     "fmc_batch_swap": (C.c_int, [C.c_void_p, C.c_ulonglong, C.c_ulonglong, C.POINTER(C.c_longlong),
                                  C.POINTER(C.c_longlong)]),
+    "fmc_batch_replica_kernel": (C.c_int, [C.c_void_p, C.c_int, I]),
     "fmc_batch_replica_info": (C.c_int, [C.c_void_p, C.c_int, D, D, C.POINTER(C.c_ulonglong),
                                          C.POINTER(C.c_ulonglong), I]),
     "fmc_batch_positions": (C.c_int, [C.c_void_p, C.c_int, D]),
@@ -542,6 +543,13 @@ class Batch:
         err = C.c_int()
         _check(lib().fmc_batch_replica_info(self.h, r, C.byref(e), C.byref(b), C.byref(m), C.byref(a), C.byref(err)))
         return dict(energy=e.value, beta=b.value, moves=m.value, accepted=a.value, error=err.value)
+
+    def kernel(self, r):
+        """The kernel that ``run`` advances replica r with: "translate" or "advance" (few or
+        many k-vectors per thread), "general", "general cells" (move sets) or "rigid"."""
+        k = C.c_int()
+        _check(lib().fmc_batch_replica_kernel(self.h, int(r), C.byref(k)))
+        return ("translate", "advance", "general", "general cells", "rigid")[k.value]
 
     def positions(self, r):
         xyz = np.zeros((self.sizes[r], 3))

@@ -589,6 +589,13 @@ int fmc_batch_replica_info(fmc_batch* b, int replica, double* energy, double* be
     });
 }
 
+int fmc_batch_replica_kernel(fmc_batch* b, int replica, int* kernel) {
+    return guarded([&] {
+        if (!kernel) throw std::runtime_error("replica_kernel: null kernel");
+        *kernel = bat(b).kernel_of(replica);
+    });
+}
+
 int fmc_batch_sample_energy(fmc_batch* b, long long every) {
     return guarded([&] { bat(b).sample_energy(every); });
 }

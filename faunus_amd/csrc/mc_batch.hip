@@ -1079,6 +1079,15 @@ void Batch::swap_counts(long long* attempted, long long* accepted) {
     *accepted = b;
 }
 
+int Batch::kernel_of(int r) {
+    if (r < 0 || r >= size()) throw std::runtime_error("replica index out of range");
+    if (!finalized_) finalize(); // which may choose the workgroup size
+    ReplicaState s = h_states_[static_cast<size_t>(r)];
+    s.parts = 1; // as in run()
+    if (general_ != 1) return translate_route(s) ? 0 : 1;
+    return rigid_route(s, fp32_ != 0) ? 4 : (s.cells ? 3 : 2);
+}
+
 ReplicaState Batch::state(int r) {
     if (r < 0 || r >= size()) throw std::runtime_error("replica index out of range");
     if (!finalized_) finalize();

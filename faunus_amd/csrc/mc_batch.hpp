@@ -314,6 +314,8 @@ class Batch {
     void sync();
     int size() const { return static_cast<int>(engines_.size()); }
     ReplicaState state(int r);
+    // kernel that run() advances replica r with (fmc_batch_replica_kernel)
+    int kernel_of(int r);
     void positions(int r, double* xyz);
     // Checkpoint of replica r: positions (3n), molecular mass centres (3 per group; may
     // be null), Philox move counter and accepted count.

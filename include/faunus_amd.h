@@ -335,6 +335,12 @@ int fmc_batch_autotune(fmc_batch* batch, long long trial_moves, int capacity, in
                        double* us_per_move, int* chosen);
 int fmc_batch_replica_info(fmc_batch* batch, int replica, double* energy, double* beta, unsigned long long* moves,
                            unsigned long long* accepted, int* error);
+/*
+ * The kernel that advances a replica in fmc_batch_run: 0 translations with few k-vectors per
+ * thread, 1 translations with more, 2 move sets without and 3 with a cell list, 4 systems of
+ * small rigid molecules (by mass centres).  No reference counterpart.
+ */
+int fmc_batch_replica_kernel(fmc_batch* batch, int replica, int* kernel);
 int fmc_batch_positions(fmc_batch* batch, int replica, double* xyz);
 int fmc_batch_trace(fmc_batch* batch, int replica, int count, int* index, unsigned char* accepted, double* du,
                     double* xyz);

@@ -22,7 +22,7 @@ def dense():  # 7.4 members per cell: 512 threads
 
 
 def water():
-    w = systems.water(n_mol=64, seed=3, kmax=4, rmax=None, cutoff=6.0)
+    w = systems.water_g2g(n_mol=64, seed=3, kmax=4, cutoff=6.0, g2g=6.0)
     return w[:5], w[5]
 
 
@@ -71,6 +71,8 @@ def test_two_workgroup_sizes_overlap():
 def test_mixed_batch_follows_the_oracle_and_its_capture(first, second, fp32):
     parts = [first(), second(), first(), second(), second()]
     b, g = batch_of(parts, fp32), batch_of(parts, fp32)
+    if first is water:
+        assert [b.kernel(r) for r in range(2)] == ["rigid", "general"]
     moves = np.array([60, 75, 0, 90, 40], np.int64)
     b.run(moves, trace=90)
     b.sync()
@@ -104,11 +106,14 @@ def test_mixed_batch_follows_the_oracle_and_its_capture(first, second, fp32):
     g.close()
 
 
-def test_server_with_jobs_of_every_kernel():
-    """The jobs of a mixed server equal the same jobs served alone."""
+@pytest.mark.parametrize("split_atoms", [0, 100])
+def test_server_with_jobs_of_every_kernel(split_atoms):
+    """The jobs of a mixed server equal the same jobs served alone, also where the chains are
+    shared by two workgroups in a cooperative launch."""
     kinds_of_job = [dilute(), dense(), water(), chain()]
+
     def serve(jobs):
-        srv = F.Server(fp32_pairs=False, max_slots=16)
+        srv = F.Server(fp32_pairs=False, max_slots=16, split_atoms=split_atoms)
         ids = [srv.submit(s, 500, seed=40 + k, kinds=m) for k, s, m in jobs]
         while srv.step(400) != (0, 0):
             pass
