@@ -48,7 +48,7 @@ __device__ __forceinline__ int cell_coord(double x, double half, double inv_cell
 }
 
 // The DevCoulomb header and the `nspl` tables in use, by all threads of the block (the whole
-// struct is 22 KB, a system without tables needs 6).
+// struct is 22.7 KB, a system without tables needs 5.7).
 __device__ __forceinline__ void copy_coulomb(DevCoulomb& dst, const DevCoulomb* __restrict__ src, int nspl, int tid,
                                              int nthreads) {
     static_assert(offsetof(DevCoulomb, spl) % 16 == 0 && sizeof(DevSplineTable) % 16 == 0, "16-byte granules");

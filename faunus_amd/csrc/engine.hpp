@@ -171,7 +171,6 @@ class Engine {
     // (reach) no pair of their atoms interacts, and below which (sure) the group cutoff
     // surely does not cut them (infinite without one).  False when there is no such reach.
     bool rigid_reach(double* reach, double* sure) const;
-    int num_columns() const { return ncol_; }
 
     // Pair-parameter and spline tables (as uploaded).
     const std::vector<DevPair>& dev_pairs() const { return h_pairs_; }

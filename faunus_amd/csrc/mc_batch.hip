@@ -439,7 +439,7 @@ ReplicaState make_replica_state(Engine& e, bool fp32, unsigned long long seed, i
     return s;
 }
 
-// Replicas with few k-vectors per thread run mc_translate_kernel, the others (K > 8 threads)
+// Replicas with at most 8 k-vectors per thread run mc_translate_kernel, the others
 // mc_advance_kernel: a function of the replica alone.
 bool translate_route(const ReplicaState& s) { return s.nk <= 8 * advance_threads(s); }
 
@@ -458,8 +458,9 @@ int advance_threads(const ReplicaState& s) {
 void launch_advance(const ReplicaState* h_states, int count, ReplicaState* d_states, const long long* d_moves, bool f32,
                     TraceEntry* trace, int trace_cap, hipStream_t stream, SideBySide& side, const LadderRun* ladders) {
     // workgroup size and kernel of each replica, functions of the replica alone (so that its
-    // arithmetic does not depend on its batch), except that the replicas of a ladder launch
-    // with cell lists take 256 threads, and the kernel for any K, when they do not agree
+    // arithmetic does not depend on the others) unless its batch set one size (the tuner, or
+    // Batch::finalize for more cell-list replicas than CUs); the replicas of a ladder launch with
+    // cell lists take 256 threads, and the kernel for any K, when they do not agree
     std::vector<int> threads(static_cast<size_t>(count));
     std::vector<char> translate(static_cast<size_t>(count));
     bool same = true, cells = true, all = true;
@@ -997,7 +998,8 @@ void Batch::replay(int count) {
 // persistent launch).  Translate-only replicas: workgroups of 256 or 512 threads (K/256
 // or K/512 k-vectors per thread; 512 holds at most 8 per thread, so K <= 4096).
 // Move-set replicas with a cell list: cells of at least the pair range (27-cell stencils)
-// or half of it (125 smaller cells).  Every candidate runs `trial` moves per replica from
+// or half of it (125 smaller cells); replicas on mc_rigid_kernel do not walk them, so for a
+// batch of these the candidates time the same kernel and either choice is as good.  Every candidate runs `trial` moves per replica from
 // checkpoints that are restored afterwards, so the chains continue from their states
 // before tuning (Q(k) and the running energy rebuilt from the positions).
 std::vector<TuneCandidate> Batch::autotune(long long trial) {

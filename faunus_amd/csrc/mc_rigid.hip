@@ -18,7 +18,13 @@
 // Per move, mc_general_kernel -> here: 4096 waters, FP32 pairs, group cutoff (8 replicas) 79.5 ->
 // 9.2 us; 1728 waters, FP64, splined and cut (4 replicas) 60.6 -> 14.0 us.  What is left is the
 // chain of a move's phases, each a few LDS or L2 latencies long at two waves per SIMD, and the
-// LDS reads of the pair energies.  1024 threads spill (36 us per move).
+// LDS reads of the pair energies.  1024 threads spill (36 us per move), and so does the form for
+// more than two k-vector pairs per thread (K above about 1900): 101 VGPRs in FP64, 173 in FP32; 100
+// moves of 4 x 1000 waters with K = 3796 take 1.6 ms there against 7.7 (FP64) on the general kernel.
+//
+// The LDS holds 16 bytes per molecule beside its tables: about 4900 molecules with FP32 pairs and
+// 5900 in FP64 (three atoms, ncut = 9); larger systems, molecules of more than 8 atoms and a cell
+// capacity fixed by the caller keep the general kernel (rigid_route, set_rigid_fields).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -100,7 +106,7 @@ __global__ __launch_bounds__(kRigidThreads) void mc_rigid_kernel(ReplicaState* _
     extern __shared__ __align__(16) unsigned char s_dyn[];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n = S.n, nk = S.nk, ncut = S.ncut, nt = S.ntypes, ng = S.ngroups;
+    const int nk = S.nk, ncut = S.ncut, nt = S.ntypes, ng = S.ngroups;
     const int w = ncut + 1;
     const RigidLds at = rigid_lds(nt, ncut, ng, nk, kF32);
     DevPair* s_pairs = reinterpret_cast<DevPair*>(s_dyn + at.pairs);
@@ -111,7 +117,6 @@ __global__ __launch_bounds__(kRigidThreads) void mc_rigid_kernel(ReplicaState* _
     uint32_t *s_cy = s_cx + pitch, *s_cz = s_cy + pitch;
     unsigned short* s_list = reinterpret_cast<unsigned short*>(s_dyn + at.list);
     const double L = S.L, half = S.half, inv = S.inv;
-    (void)n;
 
     for (int i = tid; i < nt * nt; i += kT) {
         s_pairs[i] = S.pairs[i];

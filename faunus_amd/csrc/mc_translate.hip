@@ -13,8 +13,8 @@
 //     occupancy, and the commit's cells are searched by a wave while the others sum.
 //
 // A pass of the salt ladder up to N = 8571 (48 replicas, FP32 pairs) 23.3 -> 19.2 ms against
-// mc_advance_kernel, of the one at N = 1203 (8 replicas, FP64) 5.55 -> 4.40 ms, of 800 moves of 200
-// ions with a 27-cell list (FP64) 6.03 -> 4.07 ms.  What is left at N = 8571 is the pair row (VALU
+// mc_advance_kernel, of the one at N = 1203 (8 replicas, FP64) 5.55 -> 4.38 ms, of 800 moves of 200
+// ions with a 27-cell list (FP64) 6.03 -> 3.55 ms.  What is left at N = 8571 is the pair row (VALU
 // issue at two waves per SIMD); at small N the chain of the move's phases.
 #include <hip/hip_runtime.h>
 

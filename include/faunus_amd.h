@@ -317,7 +317,8 @@ int fmc_batch_swap_counts(fmc_batch* batch, long long* attempted, long long* acc
  * the rule and deviates of fmc_batch_capture_interval).  A ladder waits only for its own
  * rungs, so ladders of different sizes run their intervals at their own pace; the rungs
  * of one ladder must share the interval count.  Translate-only replicas of one workgroup
- * size, all resident at once (an error otherwise).  Blocks until done; the swaps count
+ * size, all resident at once (an error otherwise): one per CU, or two per CU for replicas
+ * with a cell list and K <= 2048.  Blocks until done; the swaps count
  * in fmc_batch_swap_counts.  No reference counterpart as one call.
  */
 int fmc_batch_run_ladders(fmc_batch* batch, const long long* moves, const int* intervals, unsigned long long seed,
@@ -327,7 +328,8 @@ int fmc_batch_run_ladders(fmc_batch* batch, const long long* moves, const int* i
  * per replica (from checkpoints restored afterwards) and keeps the fastest for the whole
  * batch.  Candidates: 256 or 512 threads per workgroup for translate-only replicas
  * (512 when every replica has K <= 4096); cells of at least the pair range or half of it
- * (cell divisions 1 or 2) for move-set replicas with a cell list.  Writes up to
+ * (cell divisions 1 or 2) for move-set replicas with a cell list (without effect on the
+ * time of systems of small rigid molecules, fmc_batch_replica_kernel 4).  Writes up to
  * `capacity` candidates with their kernel time per replica-move (microseconds) and the
  * chosen value; num_candidates 0 means the batch has no choice.  No reference counterpart.
  */
