@@ -57,7 +57,8 @@ __device__ __forceinline__ double2 axis_phase(int n, double x, double inv) {
 // knot is then one of the four in registers.  A pair energy is bound by its LDS reads, since
 // all waves of a workgroup share one LDS: 14 reads with this window, 22 with 32 buckets per
 // table and eight knots of which one was read again (1728 FP64 waters: 3.61 -> 3.30 ms for 200
-// moves; the split kernel's 20000 Na/Cl, with the shorter phases: 3.48 -> 3.24 us per move).
+// moves; the split kernel's 20000 Na/Cl, with the shorter phases: 3.39 -> 3.23 us per move,
+// about the scatter of two builds).
 // `knots` is padded with the last knot; `coeff` is 16-byte aligned.
 __device__ __forceinline__ double spline_window(const double* __restrict__ knots, const double* __restrict__ coeff, int n,
                                                 int lo, int steps, double x) {
